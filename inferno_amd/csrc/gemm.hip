@@ -3,17 +3,14 @@
 // (dispatch_gemm_cols, kernels/gemm.mojo:198-225, called at
 // modeling/gemma_4_moe.mojo:387-392 and :485-490 with rows = HIDDEN).
 //
-// v_mfma_f32_16x16x32_bf16 with x as the A operand (16 token rows x 32 k)
-// and w as B (32 k x 16 output columns): both fragments are 16-byte runs
-// along k of one row, so w streams straight from HBM into registers and x is
-// staged once per workgroup in LDS.  A workgroup covers 64 tokens x 64
-// columns (4 waves x 16 columns, each wave up to 4 MFMA tiles down the
-// tokens) over a k range.  Decode batches (<= 64 tokens) have too few tiles
-// to fill 256 CUs: gemm_cols_split_kernel gives each workgroup a 512-wide k
-// slice loaded in one round trip and writes f32 partials that
-// gemm_cols_reduce_kernel adds in slice order.  Larger batches run
-// gemm_cols_kernel, which walks k in double-buffered 128-wide chunks (and
-// splits k the same way only while the grid is under 512 workgroups).
+// Decode batches (<= 64 tokens) stream the weight: v_mfma_f32_16x16x32_bf16
+// with x as the A operand (16 token rows x 32 k) and w as B (32 k x 16 output
+// columns), both fragments 16-byte runs along k of one row, so w goes straight
+// from HBM into registers.  They have too few output tiles to fill 256 CUs:
+// gemm_cols_split_kernel gives each workgroup a slice of k loaded in one round
+// trip and writes f32 partials that gemm_cols_reduce_kernel adds in slice
+// order.  Larger batches run gemm_cols_tile_kernel, LDS-tiled on
+// v_mfma_f32_32x32x16_bf16, in the tile shape and k splits of tile_plan.
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -22,129 +19,201 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kBM = 64;               // token rows per workgroup
-constexpr int kBN = 64;               // output columns per workgroup
-constexpr int kKC = 128;              // k per LDS chunk
-constexpr int kPitch = kKC + 8;       // LDS row pitch in bf16 (272 B: rows 4 banks apart)
-constexpr int kSegs = kBM * kKC / 8;  // 16-byte x segments per chunk
-constexpr int kSegsPerThread = kSegs / 256;
-constexpr int kMaxSplits = 16;        // k slices the reduce adds
+constexpr int kBM = 64;         // most tokens of a decode batch
+constexpr int kBN = 64;         // output columns per workgroup of a decode batch
+constexpr int kMaxSplits = 16;  // k slices the reduce adds
 
-template <bool kStream>
+// The decode batches read w once: its loads bypass the caches' retention.
 __device__ __forceinline__ uint4 load_w(const uint16_t* p) {
-  if constexpr (kStream) {
-    const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
-    return make_uint4(v.x, v.y, v.z, v.w);
-  } else {
-    return *reinterpret_cast<const uint4*>(p);
-  }
+  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// kStream: w is read by one token tile only (decode), so its loads bypass
-// the caches' retention.  kSplit: write f32 partials [split][m][n] instead of
-// bf16 outputs.
-template <bool kStream, bool kSplit>
-__global__ __launch_bounds__(256) void gemm_cols_kernel(
-    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-    uint16_t* __restrict__ out, float* __restrict__ part, int M, int N, int K,
-    int k_span) {
-  __shared__ __align__(16) uint16_t xs[2][kBM * kPitch];
-  const int wave = threadIdx.x >> 6;
+// Batches past the decode sizes: a workgroup of 4 waves (2 x 2) computes a
+// BM x BN tile of the output, walking k in 64-wide chunks that travel from
+// memory straight into LDS (global_load_lds, no registers), three chunks
+// deep: while chunk c is multiplied, c + 1 is landing and c + 2 is issued, so
+// one barrier per chunk both publishes chunk c and frees the buffer that
+// c + 2 goes to.  The three buffers are separate LDS objects, so the compiler
+// puts no wait for the loads in flight ahead of the reads of another one.
+// v_mfma_f32_32x32x16_bf16 with x as A (lane l: token l % 32, k 8*(l/32)..+7)
+// and w as B (column l % 32), so a lane stores one column of 16 tokens and 32
+// lanes 32 consecutive columns.
+//
+// LDS rows are 128 bytes (64 k); 16-byte chunk q of row r sits at q ^ ((r/2)
+// & 7), so the 16 rows that a quarter of a fragment read covers lie in 16
+// different 16-byte bank groups.
+constexpr int kTileK = 64;   // k per LDS chunk
+constexpr int kTRow = 2 * kTileK;  // LDS row bytes
+constexpr int kTThreads = 256;
+
+template <int BM, int BN, bool kSplit>
+__global__ __launch_bounds__(kTThreads) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void gemm_cols_tile_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
+    float* __restrict__ part, int M, int N, int K, int k_span, int m_tiles, int n_tiles) {
+  constexpr int kMB = BM / 64, kNB = BN / 64;  // 32 x 32 blocks of a wave's tile
+  constexpr int kLoads = (BM + BN) / 32;       // 1 KiB loads (8 rows) a wave issues per chunk
+  constexpr int kSteps = kTileK / 16;          // MFMA k steps of a chunk
+  constexpr int kStepLoads = (kLoads + kSteps - 1) / kSteps;
+  static_assert(kLoads < 16, "the wait count below");
+  __shared__ __align__(16) uint8_t buf0[(BM + BN) * kTRow];
+  __shared__ __align__(16) uint8_t buf1[(BM + BN) * kTRow];
+  __shared__ __align__(16) uint8_t buf2[(BM + BN) * kTRow];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int r = lane & 15;
-  const int g = lane >> 4;
-  const int n0 = blockIdx.x * kBN + wave * 16;
-  const int m0 = blockIdx.y * kBM;
-  const int k0 = blockIdx.z * k_span;
-  const bool live = n0 < N;  // a wave past the last column still stages x
-  const uint16_t* wp = w + static_cast<int64_t>(live ? n0 + r : 0) * K + k0 + 8 * g;
+  const int half = lane >> 5;
+  const int r32 = lane & 31;
 
-  // x staging: thread t moves segments t, t+256, ... (row s/16, 8 bf16 at
-  // 8*(s%16)); rows past M repeat row M-1 and are never stored.
-  const uint16_t* xsrc[kSegsPerThread];
-  int xdst[kSegsPerThread];
+  // Workgroups go to the 8 XCDs round robin: XCD b % 8 takes a contiguous run
+  // of tiles, ordered in bands of kBand token tiles (token tile fastest inside
+  // a band), so the 32 tiles that run together on one XCD read about as many
+  // x rows as w rows through its L2.
+  const int tiles = m_tiles * n_tiles;
+  const int per = (tiles + 7) / 8;
+  const int t = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (t >= tiles) return;  // block-uniform
+  constexpr int kBand = 1024 / BM;
+  const int band = t / (kBand * n_tiles), in_band = t - band * kBand * n_tiles;
+  const int height = min(kBand, m_tiles - band * kBand);
+  const int m0 = (band * kBand + in_band % height) * BM;
+  const int n0 = (in_band / height) * BN;
+  const int k0 = blockIdx.y * k_span;
+  const int nk = k_span / kTileK;
+
+  // Load i of this wave moves tile rows 8*(wave + 4i) .. +7 (x rows first, then
+  // w rows): lane p row p/8, LDS chunk p % 8.  Rows past the matrix repeat its
+  // last row; what they produce is not stored.
+  const uint16_t* src[kLoads];
 #pragma unroll
-  for (int i = 0; i < kSegsPerThread; ++i) {
-    const int s = threadIdx.x + 256 * i;
-    const int row = s >> 4;
-    const int col = (s & 15) * 8;
-    xsrc[i] = x + static_cast<int64_t>(min(m0 + row, M - 1)) * K + k0 + col;
-    xdst[i] = row * kPitch + col;
+  for (int i = 0; i < kLoads; ++i) {
+    const int r = 8 * (wave + 4 * i) + (lane >> 3);
+    const int chunk = (lane & 7) ^ ((r >> 1) & 7);
+    const uint16_t* base = r < BM ? x + static_cast<int64_t>(min(m0 + r, M - 1)) * K
+                                  : w + static_cast<int64_t>(min(n0 + r - BM, N - 1)) * K;
+    src[i] = base + k0 + 8 * chunk;
   }
+  auto load1 = [&](int i, int c, uint8_t* buf) {
+    __builtin_amdgcn_global_load_lds(
+        static_cast<const void*>(src[i] + static_cast<int64_t>(c) * kTileK),
+        (lds_void_t*)(buf + 8 * (wave + 4 * i) * kTRow), 16, 0, 0);
+  };
 
-  const int chunks = k_span / kKC;
-  uint4 xr[kSegsPerThread];
-  uint4 wr[kKC / 32];
+  f32x16_t acc[kMB][kNB];
 #pragma unroll
-  for (int i = 0; i < kSegsPerThread; ++i) xr[i] = *reinterpret_cast<const uint4*>(xsrc[i]);
-  if (live) {
+  for (int a = 0; a < kMB; ++a)
 #pragma unroll
-    for (int j = 0; j < kKC / 32; ++j) wr[j] = load_w<kStream>(wp + 32 * j);
-  }
+    for (int b = 0; b < kNB; ++b)
 #pragma unroll
-  for (int i = 0; i < kSegsPerThread; ++i)
-    *reinterpret_cast<uint4*>(&xs[0][xdst[i]]) = xr[i];
-  __syncthreads();
+      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
 
-  f32x4_t acc[kBM / 16];
-#pragma unroll
-  for (int t = 0; t < kBM / 16; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
+  // Fragment of 16-k step s: chunk 2s + half of row r, at (2s + half) ^ ((r/2) & 7)
+  // = 2s ^ (half ^ ((r/2) & 7)): byte offset row * 128 + (lane term ^ 32 s).
+  const int lane_sw = 16 * (half ^ ((r32 >> 1) & 7));
+  const int a_row = (wm + r32) * kTRow;
+  const int b_row = (BM + wn + r32) * kTRow;
 
-  for (int c = 0; c < chunks; ++c) {
-    const int buf = c & 1;
-    const bool more = c + 1 < chunks;
-    uint4 wn[kKC / 32];
-    if (more) {
-      const int koff = (c + 1) * kKC;
 #pragma unroll
-      for (int i = 0; i < kSegsPerThread; ++i)
-        xr[i] = *reinterpret_cast<const uint4*>(xsrc[i] + koff);
-      if (live) {
+  for (int i = 0; i < kLoads; ++i) load1(i, 0, buf0);
 #pragma unroll
-        for (int j = 0; j < kKC / 32; ++j) wn[j] = load_w<kStream>(wp + koff + 32 * j);
-      }
+  for (int i = 0; i < kLoads; ++i) load1(i, min(1, nk - 1), buf1);
+
+  auto chunk = [&](int c, const uint8_t* cur, uint8_t* next) {
+    // Chunk c has landed when only chunk c + 1's loads are outstanding.
+    __builtin_amdgcn_s_waitcnt(0x0F70 | kLoads);  // vmcnt(kLoads)
+    asm volatile("s_barrier" ::: "memory");
+    // Past the last chunk the loads repeat it into a buffer nothing reads, so
+    // the count of outstanding loads is the same in every iteration.
+    const int cn = min(c + 2, nk - 1);
+    bf16x8_t af[2][kMB], bf[2][kNB];
+    auto read = [&](int s, int set) {
+#pragma unroll
+      for (int a = 0; a < kMB; ++a)
+        af[set][a] = *reinterpret_cast<const bf16x8_t*>(cur + a_row + 32 * a * kTRow +
+                                                        (lane_sw ^ (32 * s)));
+#pragma unroll
+      for (int b = 0; b < kNB; ++b)
+        bf[set][b] = *reinterpret_cast<const bf16x8_t*>(cur + b_row + 32 * b * kTRow +
+                                                        (lane_sw ^ (32 * s)));
+    };
+    read(0, 0);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      if (s + 1 < kSteps) read(s + 1, (s + 1) & 1);
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        if (i / kStepLoads == s) load1(i, cn, next);
+#pragma unroll
+      for (int a = 0; a < kMB; ++a)
+#pragma unroll
+        for (int b = 0; b < kNB; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s & 1][a], bf[s & 1][b],
+                                                              acc[a][b], 0, 0, 0);
     }
-    if (live) {
-      const uint16_t* xb = &xs[buf][r * kPitch + 8 * g];
+    // The order within the chunk: step 0's fragment reads, then between the
+    // MFMAs of each step the reads of the next step and the step's share of
+    // the loads.
+    __builtin_amdgcn_sched_group_barrier(0x100, kMB + kNB, 0);
 #pragma unroll
-      for (int j = 0; j < kKC / 32; ++j) {
-        const bf16x8_t b = __builtin_bit_cast(bf16x8_t, wr[j]);
+    for (int s = 0; s < kSteps; ++s) {
+      constexpr int kMfma = kMB * kNB, kReads = kMB + kNB;
+      int reads = 0, loads = 0;
 #pragma unroll
-        for (int t = 0; t < kBM / 16; ++t) {
-          const uint4 av = *reinterpret_cast<const uint4*>(xb + 16 * t * kPitch + 32 * j);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), b,
-                                                           acc[t], 0, 0, 0);
+      for (int j = 0; j < kMfma; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (s + 1 < kSteps) {
+          constexpr int kPer = (kReads + kMfma - 1) / kMfma;
+#pragma unroll
+          for (int t = 0; t < kPer; ++t)
+            if (reads < kReads) {
+              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+              ++reads;
+            }
         }
+        constexpr int kPerL = (kStepLoads + kMfma - 1) / kMfma;
+#pragma unroll
+        for (int t = 0; t < kPerL; ++t)
+          if (loads < kStepLoads && s * kStepLoads + loads < kLoads) {
+            __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+            ++loads;
+          }
       }
     }
-    if (more) {
-#pragma unroll
-      for (int i = 0; i < kSegsPerThread; ++i)
-        *reinterpret_cast<uint4*>(&xs[buf ^ 1][xdst[i]]) = xr[i];
-#pragma unroll
-      for (int j = 0; j < kKC / 32; ++j) wr[j] = wn[j];
-    }
-    __syncthreads();
+  };
+  int c = 0;
+  for (; c + 3 <= nk; c += 3) {
+    chunk(c, buf0, buf2);
+    chunk(c + 1, buf1, buf0);
+    chunk(c + 2, buf2, buf1);
   }
+  if (c < nk) chunk(c, buf0, buf2);
+  if (c + 1 < nk) chunk(c + 1, buf1, buf0);
+  // No load may still be on its way into LDS when the workgroup ends.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  if (!live) return;
-  // C layout: acc[t][j] is token m0 + 16t + 4g + j, column n0 + r.
+  // C layout: value 4j + i of a block is token 8j + 4*half + i, column r32.
 #pragma unroll
-  for (int t = 0; t < kBM / 16; ++t) {
+  for (int a = 0; a < kMB; ++a)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = m0 + 16 * t + 4 * g + j;
-      if (m >= M) continue;
-      const int64_t o = static_cast<int64_t>(m) * N + n0 + r;
-      if constexpr (kSplit) {
-        part[static_cast<int64_t>(blockIdx.z) * M * N + o] = acc[t][j];
-      } else {
-        out[o] = static_cast<uint16_t>(f32_to_bf16_bits(acc[t][j]));
+    for (int b = 0; b < kNB; ++b) {
+      const int n = n0 + wn + 32 * b + r32;
+      if (n >= N) continue;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + wm + 32 * a + 8 * (v >> 2) + 4 * half + (v & 3);
+        if (m >= M) continue;
+        const int64_t o = static_cast<int64_t>(m) * N + n;
+        if constexpr (kSplit)
+          part[static_cast<int64_t>(blockIdx.y) * M * N + o] = acc[a][b][v];
+        else
+          out[o] = static_cast<uint16_t>(f32_to_bf16_bits(acc[a][b][v]));
       }
     }
-  }
 }
 
 // Decode batches (M <= 64 tokens): one workgroup takes 64 columns and one
@@ -171,7 +240,7 @@ __global__ __launch_bounds__(256) void gemm_cols_split_kernel(
   if (live) {
     const uint16_t* wp = w + static_cast<int64_t>(n0 + r) * K + k0 + 8 * g;
 #pragma unroll
-    for (int j = 0; j < kSpan / 32; ++j) wr[j] = load_w<true>(wp + 32 * j);
+    for (int j = 0; j < kSpan / 32; ++j) wr[j] = load_w(wp + 32 * j);
   }
   uint4 xr[kXSegs];
 #pragma unroll
@@ -261,17 +330,76 @@ int decode_span(int64_t M, int64_t K) {
   return 0;
 }
 
+template <int BM, int BN>
+hipError_t launch_tile(const uint16_t* x, const uint16_t* w, uint16_t* out, float* part, int M,
+                       int N, int K, int splits, hipStream_t stream) {
+  const int mt = (M + BM - 1) / BM, nt = (N + BN - 1) / BN;
+  const unsigned blocks = static_cast<unsigned>((mt * nt + 7) / 8) * 8;
+  const dim3 grid(blocks, static_cast<unsigned>(splits));
+  if (splits > 1)
+    hipLaunchKernelGGL((gemm_cols_tile_kernel<BM, BN, true>), grid, dim3(kTThreads), 0, stream,
+                       x, w, out, part, M, N, K, K / splits, mt, nt);
+  else
+    hipLaunchKernelGGL((gemm_cols_tile_kernel<BM, BN, false>), grid, dim3(kTThreads), 0, stream,
+                       x, w, out, nullptr, M, N, K, K, mt, nt);
+  return hipGetLastError();
+}
+
+// Tile shape and k splits of a batch past the decode sizes: the cheapest by a
+// model of the launch fitted to sweeps of every shape and split over 65 to
+// 16,384 tokens at N = 2816, K = 4096 and 8192.  A tile costs `us` per 1,024 of
+// k and the card runs 256 of them at a time (the 64 x 64 tile three per CU, so
+// its partial rounds cost their share only); splits add the reduce launch,
+// their own start and the f32 partials' way out and back.  It picks the
+// measured best or one within 5 % of it (12 % at 128 tokens): 128 x 128 in two
+// splits 21.8 us at 500 tokens, 192 x 128 45.1 us at 2,000 (242 of 256 CUs;
+// 256 x 128, 176 tiles, 47.9), 256 x 128 342 us at 16,384 (1,106 TFLOP/s).
+struct TilePlan {
+  int bm, bn, splits;
+};
+TilePlan tile_plan(int64_t M, int64_t N, int64_t K) {
+  struct Shape {
+    int bm, bn;
+    double us;
+  };
+  constexpr Shape kShapes[] = {
+      {256, 128, 11.6}, {192, 128, 9.4}, {128, 128, 6.9}, {128, 64, 5.0}, {64, 64, 4.0}};
+  TilePlan best{256, 128, 1};
+  double best_us = 1e30;
+  for (const Shape& sh : kShapes) {
+    const int64_t tiles = ((M + sh.bm - 1) / sh.bm) * ((N + sh.bn - 1) / sh.bn);
+    for (int splits = 1; splits <= kMaxSplits; splits *= 2) {
+      if ((K / 128) % splits != 0 || (splits > 1 && tiles * splits > 512)) break;
+      const double load = static_cast<double>(tiles * splits) / 256.0;
+      const double rounds =
+          sh.bm == 64 ? (load > 1.0 ? load : 1.0) : static_cast<double>((tiles * splits + 255) / 256);
+      double us = rounds * sh.us * static_cast<double>(K / splits) / 1024.0;
+      if (splits > 1) us += 4.0 + 0.4 * splits + static_cast<double>(splits) * M * N / 1e6;
+      if (us < best_us) {
+        best_us = us;
+        best = {sh.bm, sh.bn, splits};
+      }
+    }
+  }
+  return best;
+}
+
+hipError_t launch_plan(const TilePlan& p, const uint16_t* x, const uint16_t* w, uint16_t* out,
+                       float* part, int M, int N, int K, hipStream_t stream) {
+  if (p.bm == 256) return launch_tile<256, 128>(x, w, out, part, M, N, K, p.splits, stream);
+  if (p.bm == 192) return launch_tile<192, 128>(x, w, out, part, M, N, K, p.splits, stream);
+  if (p.bm == 128 && p.bn == 128)
+    return launch_tile<128, 128>(x, w, out, part, M, N, K, p.splits, stream);
+  if (p.bm == 128) return launch_tile<128, 64>(x, w, out, part, M, N, K, p.splits, stream);
+  return launch_tile<64, 64>(x, w, out, part, M, N, K, p.splits, stream);
+}
+
 }  // namespace
 
 int gemm_cols_splits(int64_t M, int64_t N, int64_t K) {
   const int span = decode_span(M, K);
   if (span) return static_cast<int>(K / span);
-  const int64_t tiles = ((N + kBN - 1) / kBN) * ((M + kBM - 1) / kBM);
-  const int64_t chunks = K / kKC;
-  int splits = 1;
-  while (tiles * splits * 2 <= 512 && chunks % (splits * 2) == 0 && splits * 2 <= kMaxSplits)
-    splits *= 2;
-  return splits;
+  return tile_plan(M, N, K).splits;
 }
 
 int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K) {
@@ -284,17 +412,14 @@ hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* work
                             int64_t M, int64_t N, int64_t K, hipStream_t stream) {
   if (M <= 0) return hipSuccess;
   const int splits = gemm_cols_splits(M, N, K);
-  const int k_span = static_cast<int>(K / splits);
-  dim3 grid(static_cast<unsigned>((N + kBN - 1) / kBN),
-            static_cast<unsigned>((M + kBM - 1) / kBM), static_cast<unsigned>(splits));
   const auto* xp = static_cast<const uint16_t*>(x);
   const auto* wp = static_cast<const uint16_t*>(w);
   auto* op = static_cast<uint16_t*>(out);
-  const bool stream_w = grid.y == 1;
+  const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  hipError_t err;
   if (const int span = decode_span(M, K)) {
-    dim3 sgrid(grid.x, static_cast<unsigned>(splits));
+    dim3 sgrid(static_cast<unsigned>((N + kBN - 1) / kBN), static_cast<unsigned>(splits));
     const int tm = static_cast<int>((M + 15) / 16);
-    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
     if (span == 256) {  // M <= 16
       hipLaunchKernelGGL((gemm_cols_split_kernel<1, 256>), sgrid, dim3(256), 0, stream, xp,
                          wp, workspace, m, n, k);
@@ -311,33 +436,13 @@ hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* work
       hipLaunchKernelGGL((gemm_cols_split_kernel<4, 512>), sgrid, dim3(256), 0, stream, xp,
                          wp, workspace, m, n, k);
     }
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    return launch_reduce_n<1>(workspace, op, M * N / 4, M * N, splits, stream);
-  }
-  if (splits > 1) {
-    if (stream_w) {
-      hipLaunchKernelGGL((gemm_cols_kernel<true, true>), grid, dim3(256), 0, stream, xp, wp,
-                         op, workspace, static_cast<int>(M), static_cast<int>(N),
-                         static_cast<int>(K), k_span);
-    } else {
-      hipLaunchKernelGGL((gemm_cols_kernel<false, true>), grid, dim3(256), 0, stream, xp, wp,
-                         op, workspace, static_cast<int>(M), static_cast<int>(N),
-                         static_cast<int>(K), k_span);
-    }
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    return launch_reduce_n<1>(workspace, op, M * N / 4, M * N, splits, stream);
-  } else if (stream_w) {
-    hipLaunchKernelGGL((gemm_cols_kernel<true, false>), grid, dim3(256), 0, stream, xp, wp, op,
-                       nullptr, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
-                       k_span);
+    err = hipGetLastError();
   } else {
-    hipLaunchKernelGGL((gemm_cols_kernel<false, false>), grid, dim3(256), 0, stream, xp, wp,
-                       op, nullptr, static_cast<int>(M), static_cast<int>(N),
-                       static_cast<int>(K), k_span);
+    err = launch_plan(tile_plan(M, N, K), xp, wp, op, workspace, m, n, k, stream);
+    if (splits == 1) return err;
   }
-  return hipGetLastError();
+  if (err != hipSuccess) return err;
+  return launch_reduce_n<1>(workspace, op, M * N / 4, M * N, splits, stream);
 }
 
 }  // namespace ifr

@@ -61,6 +61,23 @@ def test_gemm_cols_integer_operands_bit_exact(seq, rows, cols):
     assert np.array_equal(got, want)
 
 
+# Sizes around every tile shape of the batched kernel (64, 128, 192 and 256
+# tokens by 64 or 128 columns), its k splits and its three-chunk loop (2, 4, 6
+# and 64 chunks): integer operands, so every sum is exact in any order.
+@pytest.mark.parametrize("seq,rows,cols", [(65, 16, 128), (65, 2816, 4096), (127, 144, 256),
+                                           (129, 80, 384), (193, 2816, 512), (500, 2816, 4096),
+                                           (769, 2816, 256), (1537, 2816, 128),
+                                           (2000, 2816, 384), (4099, 1040, 128)])
+def test_gemm_cols_tiles_bit_exact(seq, rows, cols):
+    announce(f"gemm_cols tiles seq={seq} rows={rows} cols={cols}")
+    rng = np.random.default_rng(seq + rows + cols)
+    x = rng.integers(-3, 4, (seq, cols)).astype(np.float32)
+    w = rng.integers(-3, 4, (rows, cols)).astype(np.float32)
+    got = _run(_bf(x), _bf(w), seq, rows, cols)
+    # |sum| <= 9 * 4096: exact in f32, and one rounding to bf16 in the oracle's conversion.
+    assert np.array_equal(got, oracle.f32_to_bf16((x @ w.T).ravel()).reshape(seq, rows))
+
+
 def test_gemm_cols_rejects_unsupported_shapes():
     from inferno_amd._lib import InfernoHipError
 
