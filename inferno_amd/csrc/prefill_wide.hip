@@ -298,6 +298,12 @@ void prefill_wide_mfma_kernel(
 
   if (n_iters > 0) stage(0, kbuf0, vbuf0, 0);
   __builtin_amdgcn_s_waitcnt(0);
+  // The Q^T fragments are waited for here.  Otherwise the compiler moves their
+  // loads past the wait, carries them as outstanding into the loop, and puts a
+  // vmcnt(0) among the score MFMAs of every iteration, right behind the first
+  // staging load of the next one.
+#pragma unroll
+  for (int d = 0; d < kQFrags; ++d) asm volatile("" : "+v"(qf[d]));
   if (n_iters > 0) land_v(0, vbuf0);
   __syncthreads();
 
