@@ -746,6 +746,21 @@ int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
   // The MFMA prefill routes finalise in-kernel and write no partials.
   if (route == PrefillRoute::kNone && partials_bytes < info[3] * partial_stride * 4)
     return fail(IFR_ESPACE, "partials need %lld bytes", (long long)(info[3] * partial_stride * 4));
+  if (route == PrefillRoute::kFull256 || route == PrefillRoute::kWide512) {
+    const int kind =
+        ifr::prefill_narrow_kind(info[14], info[6], info[5], num_kv, static_cast<int>(head_dim),
+                                 kv_stride, static_cast<int>(pow2_shift(page_len)));
+    if (kind) {
+      // Few rows (a short chunk, or tokens decoding beside one).
+      IFR_HIP(ifr::launch_prefill_narrow(static_cast<const int32_t*>(image_dev), kind,
+                                         static_cast<int>(info[14]), q, k_base, v_base, output,
+                                         static_cast<int>(head_dim), static_cast<int>(num_q),
+                                         static_cast<int>(num_kv), kv_stride, g,
+                                         as_stream(stream)),
+              "prefill_narrow");
+      return ok();
+    }
+  }
   if (route == PrefillRoute::kFull256) {
     // Prefill chunk of full attention: MFMA query blocks, finalised in-kernel.
     IFR_HIP(ifr::launch_prefill_full_mfma(static_cast<const int32_t*>(image_dev),

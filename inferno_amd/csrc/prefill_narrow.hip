@@ -2,25 +2,39 @@
 // walk as the query-block kernels (FlashPrefillFullKernel + PrefillMergeKernel,
 // kernels/flash_attention_prefill.mojo:117-248: tiles of 16 keys from key 0,
 // the biased exp, one-segment merge), split over the waves of a workgroup so
-// that 32 rows (tokens x the q heads of one kv head) occupy a whole CU.
+// that 32 rows (tokens x the q heads of one kv head) take four waves.
 //
 // A query-block kernel gives each wave 32 rows and all keys: a chunk of 512
-// tokens is 64 blocks on 256 CUs, and one decoding token's block walks its
-// keys with 2 of 128 rows live.  Here the NW waves of a block share 32 rows:
+// tokens is 64 blocks on 256 CUs, and a decoding token's block in a mixed step
+// walks its keys with 2 of 128 rows live.  Here the four waves of a block share
+// 32 rows:
 //
-//   scores   wave w forms the NW-tile iteration's tile w:
-//            S (16 keys x 32 rows) = K . Q^T      v_mfma_f32_16x16x32_bf16
+//   scores   each wave takes its own 16-key tile(s) of the iteration, S = K . Q^T
 //   softmax  the tile maxima go through LDS; every wave then knows the running
 //            maximum before and after each tile of the iteration, so all tiles
 //            of it take their weights at once, scaled by the product of the
 //            later tiles' corrections
-//   P.V      wave w owns D / NW output dims of all 32 rows and reads every
-//            wave's weights (bf16 hi + lo parts) from LDS:
-//            O^T (16 dims x 32 rows) += V^T . P^T
+//   P.V      each wave owns a quarter of the output dims and reads every wave's
+//            weights (bf16 hi + lo parts) from LDS, O^T += V^T . P^T
 //
 // K tiles and V column slices are private to the wave that multiplies them, so
 // it refills them (global_load_lds) as soon as it has read them, without a
 // barrier; the two barriers of an iteration publish the maxima and the weights.
+//
+// What bounds them is instruction issue: a lone wave of a SIMD issues about one
+// instruction per 5 cycles and one LDS read per 24 to 34.  Hence two kernels.
+// prefill_narrow_pairs_kernel (head_dim 256) takes tile pairs on
+// v_mfma_f32_32x32x16_bf16, 128 keys an iteration: the fewest instructions per
+// key, but its LDS fills a CU.  prefill_narrow_tiles_kernel takes single tiles
+// on v_mfma_f32_16x16x32_bf16, 64 keys an iteration: two blocks fit a CU at
+// head_dim 256 and run under each other's waits.
+//
+// Measured at 16 q / 8 kv heads x 256 (us, the query-block kernel / pairs /
+// tiles): 64 tokens on 7,000 296 / 134 / 185; 500 on 7,013 484 / 140 / 192;
+// 1,000 on 7,000 513 / 278 / 250; 2,000 on 7,000 552 / 580 / 505; 32 tokens
+// decoding at 3,000 beside a 512-token chunk 374 / 191 / 157.  At 16 / 2 x 512
+// (query-block kernel / tiles): 64 tokens 518 / 275; 500 690 / 300; 1,000 750 /
+// 580; 2,000 671 / 1,230; the mixed step 630 / 290.
 #include <type_traits>
 
 #include "launch.hpp"
@@ -32,9 +46,11 @@ namespace {
 using namespace prefill;
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kNRows = 32;         // rows of a block
-constexpr int kRG = kNRows / 16;   // 16-row groups
+constexpr int kNRows = 32;        // rows of a block
+constexpr int kRG = kNRows / 16;  // 16-row groups
+constexpr int kNW = 4;            // waves of a block
 
 // Members of the (lane, lane ^ 16) and (lane, lane ^ 32) pairs, lower lane
 // first, the same in both lanes.
@@ -50,6 +66,19 @@ __device__ __forceinline__ void pair32(float x, float& lo, float& hi) {
   lo = __uint_as_float(r[0]);
   hi = __uint_as_float(r[1]);
 }
+__device__ __forceinline__ float raw_max(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// Over the four 16-lane groups.
+__device__ __forceinline__ float groups_max(float x) {
+  float a, b;
+  pair16(x, a, b);
+  x = raw_max(a, b);
+  pair32(x, a, b);
+  return raw_max(a, b);
+}
 __device__ __forceinline__ float groups_mul(float x) {
   float a, b;
   pair16(x, a, b);
@@ -64,14 +93,88 @@ __device__ __forceinline__ float groups_add(float x) {
   pair32(x, a, b);
   return a + b;
 }
-__device__ __forceinline__ float raw_max(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+
+// 1 KiB loads into LDS: load i goes to lds (wave-uniform) + 1024 i + 16 * lane,
+// from base (wave-uniform) + off_i + 1024 i (the instruction's offset counts on
+// both sides; off_i is unsigned, so callers keep base low enough).  As
+// instructions the compiler does not track: its tracking of such loads stops at
+// the transposing LDS reads, which carry no alias information, and would wait
+// there for every load in flight.  The waits are written out below (loads return
+// in order, so the ones the compiler adds for its own loads can only wait for
+// more).  m0 is put back, as the compiler does not know of the change.
+__device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)p));
+}
+__device__ __forceinline__ void load_lds4(const char* base, uint32_t o0, uint32_t o1, uint32_t o2,
+                                          uint32_t o3, const uint8_t* lds) {
+  uint32_t m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\t"
+      "global_load_lds_dwordx4 %2, %6\n\t"
+      "global_load_lds_dwordx4 %3, %6 offset:1024\n\t"
+      "global_load_lds_dwordx4 %4, %6 offset:2048\n\t"
+      "global_load_lds_dwordx4 %5, %6 offset:3072\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(m0)
+      : "s"(lds_addr(lds)), "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(base)
+      : "memory");
+}
+__device__ __forceinline__ void load_lds2(const char* base, uint32_t o0, uint32_t o1,
+                                          const uint8_t* lds) {
+  uint32_t m0;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\t"
+      "global_load_lds_dwordx4 %2, %4\n\t"
+      "global_load_lds_dwordx4 %3, %4 offset:1024\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(m0)
+      : "s"(lds_addr(lds)), "v"(o0), "v"(o1), "s"(base)
+      : "memory");
 }
 
-// s_waitcnt operand that waits for vmcnt <= n alone.
-constexpr int vmcnt_only(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+// The sub-block (kTok tokens of a plan query block) that block number `rest`
+// takes, counting only those with tokens, in plan order and the longest key
+// range of a query block first: qb (-1 past the last) and sub.  The blocks
+// without one then all come last.  (A grid of every query block's sub-blocks in
+// order puts the single live one of each decoding token's query block on the
+// same shader engine: 64 of 256 CUs did that work.)
+template <int kTok>
+__device__ __forceinline__ void pick_sub_block(const int32_t* image, int rest, int& qb, int& sub) {
+  const int n_qb = image[kHdrNumQBlocks];
+  const int32_t* blocks = image + image[kHdrOffQBlocks];
+  const int lane = threadIdx.x & 63;
+  qb = -1;
+  sub = 0;
+  for (int first = 0; first < n_qb; first += 64) {
+    const int i = first + lane;
+    const int cnt = i < n_qb ? (blocks[i * kQBlockWords + 2] + kTok - 1) / kTok : 0;
+    int x = cnt;  // inclusive scan over the wave
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31
+    const int total = __builtin_amdgcn_readlane(x, 63);
+    if (rest < total) {  // wave-uniform
+      const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64(x > rest));
+      qb = first + l;
+      sub = __builtin_amdgcn_readlane(x, l) - 1 - rest;
+      return;
+    }
+    rest -= total;
+  }
+}
+
+// Waits until at most n loads are outstanding.  The memory clobber keeps the LDS
+// reads of what they bring behind it.
+template <int n>
+__device__ __forceinline__ void wait_loads() {
+  if constexpr (n == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  else if constexpr (n == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  else if constexpr (n == 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  else static_assert(n == 0, "a count with an instruction");
+}
 
 // LDS written so far is visible to the block; the loads in flight stay in
 // flight (a __syncthreads would wait for them).
@@ -79,18 +182,17 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <int D, int G, int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4)))
-void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __restrict__ q,
+template <int D, int G, int kPerSimd>
+__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(kPerSimd, kPerSimd)))
+void prefill_narrow_tiles_kernel(const int32_t* __restrict__ image, const uint16_t* __restrict__ q,
                            const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
                            uint16_t* __restrict__ out, int num_q, int num_kv,
                            int64_t kv_stride, int shift, int row_mask) {
   constexpr int kTok = kNRows / G;                // tokens of a block
-  constexpr int kSub = kPrefillTokens / kTok;     // blocks per plan query block
-  constexpr int kKI = 16 * NW;                    // keys per iteration
+  constexpr int kKI = 16 * kNW;                    // keys per iteration
   constexpr int kRowB = 2 * D;                    // bytes of a K row in LDS
   constexpr int kKS = D / 32;                     // score MFMA steps
-  constexpr int kDW = D / NW;                     // output dims of a wave
+  constexpr int kDW = D / kNW;                     // output dims of a wave
   constexpr int kDB = kDW / 16;                   // 16-dim blocks of it
   constexpr int kVB = 2 * kDW;                    // bytes of a V row slice in LDS
   constexpr int kPS = kKI / 32;                   // P.V MFMA steps
@@ -99,17 +201,16 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
   constexpr int kKRowsPerLoad = 1024 / kRowB;     // 2 (D = 256) or 1
   constexpr int kLPK = kVB / 16;                  // lanes per V row slice
   constexpr int kKPL = 64 / kLPK;                 // V rows per load
-  constexpr int kVLoads = kKI / kKPL;
-  constexpr int kTPG = NW / 4;                    // tiles per 16-lane group
-  static_assert(kKLoads < 16 + 1 && kVLoads < 16 + 1 && kTPG >= 1 && kTPG <= 2, "shape");
+  static_assert(kKS % kNW == 0 && kKLoads % 4 == 0, "shape");
 
-  __shared__ __align__(16) uint8_t kbuf[NW * 16 * kRowB];
-  __shared__ __align__(16) uint8_t vbuf[NW * kKI * kVB];
+  __shared__ __align__(16) uint8_t kbuf[kNW * 16 * kRowB];
+  __shared__ __align__(16) uint8_t vbuf[kNW * kKI * kVB];
   __shared__ __align__(16) uint8_t phi[kNRows * kPRow];
   __shared__ __align__(16) uint8_t plo[kNRows * kPRow];
-  __shared__ __align__(16) float tmax[kNRows][NW];
-  __shared__ __align__(16) float tsum[kNRows][NW];
-  __shared__ __align__(16) int32_t big_flag[NW];
+  __shared__ __align__(16) float tmax[kNRows][kNW];
+  __shared__ __align__(16) float tsum[kNRows][kNW];
+  __shared__ __align__(16) int32_t big_flag[kNW];
+  __shared__ float unused[64];
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -117,12 +218,12 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
   const int grp = lane >> 4;
   const int g = blockIdx.x % num_kv;
   const int rest = blockIdx.x / num_kv;
-  const int qb = rest / kSub;
-  const int sub = kSub - 1 - rest % kSub;  // the longest key range first
+  int qb, sub;
+  pick_sub_block<kTok>(image, rest, qb, sub);
+  if (qb < 0) return;  // block-uniform
 
   const int32_t* blk = image + image[kHdrOffQBlocks] + qb * kQBlockWords;
   const int run = blk[0];
-  if (sub * kTok >= blk[2]) return;  // block-uniform
   const int t0 = blk[1] + sub * kTok;
   const int ntok = min(kTok, blk[2] - sub * kTok);
   const int32_t* rp = image + image[kHdrOffRuns] + run * 4;
@@ -163,53 +264,64 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
   const char* kg = reinterpret_cast<const char*>(kc + static_cast<int64_t>(g) * D);
   const char* vg = reinterpret_cast<const char*>(vc + static_cast<int64_t>(g) * D + wave * kDW);
   auto v_swz = [](int key) -> int {
-    if constexpr (kVB == 64) return (key >> 3) & 1;
-    else if constexpr (kVB == 128) return ((key >> 1) & 1) | (((key >> 3) & 1) << 1);
+    if constexpr (kVB == 128) return ((key >> 1) & 1) | (((key >> 3) & 1) << 1);
     else return (key & 3) | (((key >> 3) & 1) << 2);
   };
   // First cache rows of the tiles of iteration it, tile t in lane t (pages hold
   // whole tiles: page_len >= 16); tiles past the last one repeat it.  Loaded an
   // iteration before the staging that uses them.
   auto tile_slots = [&](int it) -> int {
-    const int key = 16 * min(it * NW + (lane & (NW - 1)), last_tile);
+    const int key = 16 * min(it * kNW + (lane & (kNW - 1)), last_tile);
     return rows[key >> shift] + (key & row_mask);
   };
-  auto slot_of = [&](int slots, int t) -> int64_t {
-    return __builtin_amdgcn_readlane(slots, t);
+  auto slot_of = [&](int sl, int t) -> int64_t {
+    return __builtin_amdgcn_readlane(sl, t);
   };
+  // The K tile is 16 rows in kKLoads loads, 4 at a time: row kKRowsPerLoad * i +
+  // k_lrow of load i, its chunk ^ the row.  Rows past the block's last key are
+  // other rows of its page; their scores are masked.
   const int k_lrow = lane / (64 / kKRowsPerLoad);
-  const uint32_t k_off = static_cast<uint32_t>(k_lrow) * static_cast<uint32_t>(row_bytes);
-  const uint32_t k_chunk = 16u * static_cast<uint32_t>((lane % (64 / kKRowsPerLoad)) ^ k_lrow);
-  auto stage_k = [&](int slots) {
-    // Rows past the block's last key are other rows of its page; their scores
-    // are masked.
-    const char* kb = kg + slot_of(slots, wave) * row_bytes;
+  const uint32_t rb32 = static_cast<uint32_t>(row_bytes);
+  uint32_t k_off[kKLoads];
 #pragma unroll
-    for (int i = 0; i < kKLoads; ++i)  // chunk ^ row, row = kKRowsPerLoad * i + k_lrow
-      __builtin_amdgcn_global_load_lds(
-          static_cast<const void*>(kb + i * kKRowsPerLoad * row_bytes +
-                                   (k_off + (k_chunk ^ (16u * kKRowsPerLoad * i)))),
-          (lds_void_t*)(kw + i * 1024), 16, 0, 0);
+  for (int i = 0; i < kKLoads; ++i) {
+    const int row = kKRowsPerLoad * i + k_lrow;
+    k_off[i] = static_cast<uint32_t>(row) * rb32 +
+               16u * static_cast<uint32_t>((lane % (64 / kKRowsPerLoad)) ^ row) +
+               1024u * (3 - i % 4);
+  }
+  auto stage_k4 = [&](int i4, const char* kb) {
+    const int i = 4 * i4;
+    load_lds4(kb - 3072, k_off[i], k_off[i + 1], k_off[i + 2], k_off[i + 3], kw + i * 1024);
   };
+  auto k_base = [&](int sl) { return kg + slot_of(sl, wave) * row_bytes; };
+  // Tile t of the wave's V slice of iteration it, 16 rows in kVT loads.  tail:
+  // the iteration may reach past the last key; keys past it repeat a valid row
+  // (their weights are 0, and its values finite).
+  constexpr int kVT = 16 / kKPL;
+  static_assert(kVT == 2 || kVT == 4, "V loads of a tile");
   const int v_lrow = lane / kLPK;
-  const int v_lchunk = lane % kLPK;
-  // kTail: the iteration may reach past the last key; keys past it repeat a
-  // valid row (their weights are 0, and its values finite).
-  auto stage_v = [&](auto tail, int it, int slots) {
+  uint32_t v_chunk[kVT], v_off[kVT];  // the swizzle repeats every 16 keys
 #pragma unroll
-    for (int i = 0; i < kVLoads; ++i) {
-      const int k0 = i * kKPL;  // first key of the load within the iteration
-      int lrow = v_lrow;
+  for (int i = 0; i < kVT; ++i) {
+    const int row = kKPL * i + v_lrow;
+    v_chunk[i] = 16u * static_cast<uint32_t>((lane % kLPK) ^ (2 * v_swz(row))) + 1024u * (kVT - 1 - i);
+    v_off[i] = static_cast<uint32_t>(row) * rb32 + v_chunk[i];
+  }
+  auto stage_v = [&](auto tail, int t, int it, int sl) {
+    const char* vb = vg + slot_of(sl, t) * row_bytes - 1024 * (kVT - 1);
+    uint32_t off[kVT];
+#pragma unroll
+    for (int i = 0; i < kVT; ++i) {
+      off[i] = v_off[i];
       if constexpr (tail.value) {
-        const int tile = min(it * NW + k0 / 16, last_tile);
-        lrow = min(lrow, count_max - 1 - 16 * tile - (k0 & 15));
+        const int last = count_max - 1 - 16 * min(it * kNW + t, last_tile);
+        off[i] = static_cast<uint32_t>(min(kKPL * i + v_lrow, last)) * rb32 + v_chunk[i];
       }
-      const char* vb = vg + (slot_of(slots, k0 / 16) + (k0 & 15)) * row_bytes;
-      const int64_t off = static_cast<int64_t>(lrow) * row_bytes +
-                          16 * (v_lchunk ^ (2 * v_swz(k0 + v_lrow)));
-      __builtin_amdgcn_global_load_lds(static_cast<const void*>(vb + off),
-                                       (lds_void_t*)(vw + i * 1024), 16, 0, 0);
     }
+    const uint8_t* dst = vw + t * kVT * 1024;
+    if constexpr (kVT == 2) load_lds2(vb, off[0], off[1], dst);
+    else load_lds4(vb, off[0], off[1], off[2], off[3], dst);
   };
 
   // ---- per-row state, the same in the four lanes of a row ----
@@ -223,24 +335,38 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
 #pragma unroll
     for (int b = 0; b < kDB; ++b) acc[b][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  int slots = tile_slots(0);  // of the next iteration to stage
-  stage_k(slots);
-  stage_v(std::true_type{}, 0, slots);
-  slots = tile_slots(min(1, n_it - 1));
+  int slots = tile_slots(0);                      // of the iteration at hand
+  int slots_next = tile_slots(min(1, n_it - 1));  // and of the one after it
+#pragma unroll
+  for (int i = 0; i < kKLoads / 4; ++i) stage_k4(i, k_base(slots));
 
-  const int p_swz_row = kPRow == 256 ? r16 : (r16 >> 1) & 7;  // chunk swizzle of a P row
+  const int p_swz_row = (r16 >> 1) & 7;  // chunk swizzle of a P row (128 bytes)
   const int k_read = r16 * kRowB;
   // Transposing read of dim block b, keys 32 s + 8 grp + 0..3 (+4): lane j of a
   // 16-lane group addresses key j / 4 of them, dims 4 (j % 4) .. +3.
   const int vkey = 8 * grp + (r16 >> 2);
 
-  // One iteration.  general: some rows may end inside it, or the next one may
-  // reach past the last key.
+  // Where the lanes of group 0 publish a row's value; the other lanes write to
+  // an unused place instead of branching.
+  float* pub_max[kRG];
+  float* pub_sum[kRG];
+#pragma unroll
+  for (int i = 0; i < kRG; ++i) {
+    pub_max[i] = grp == 0 ? &tmax[16 * i + r16][wave] : &unused[lane];
+    pub_sum[i] = grp == 0 ? &tsum[16 * i + r16][wave] : &unused[lane];
+  }
+  int p_write[kRG];
+#pragma unroll
+  for (int i = 0; i < kRG; ++i)
+    p_write[i] = (16 * i + r16) * kPRow + 16 * ((2 * wave + (grp >> 1)) ^ p_swz_row) + 8 * (grp & 1);
+
+  // One iteration.  general: some rows may end inside it.
   auto iteration = [&](auto general, int it) {
     constexpr bool kGeneral = general.value;
-    const int itn = min(it + 1, n_it - 1);
-    // ---- scores of tile it * NW + wave ----
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(kVLoads));  // K landed
+    const int tile0 = (it * kNW + wave) * 16;
+    // ---- scores of tile it * kNW + wave, with the V loads of the iteration
+    // between the MFMAs (its slice was read by the last P.V) ----
+    wait_loads<0>();  // K landed
     f32x4_t sc[kRG];
     {
       bf16x8_t kf[kKS];
@@ -250,21 +376,16 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
 #pragma unroll
       for (int i = 0; i < kRG; ++i) sc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int s = 0; s < kKS; ++s)
+      for (int s = 0; s < kKS; ++s) {
+        if (s % (kKS / kNW) == 0) stage_v(general, s / (kKS / kNW), it, slots);
 #pragma unroll
         for (int i = 0; i < kRG; ++i)
           sc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s], qf[i][s], sc[i], 0, 0, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, kKS, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, kKS * kRG, 0);
+      }
     }
-    // The tile's rows are in registers: refill the buffer.
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    const int slots_after = tile_slots(min(it + 2, n_it - 1));
-    stage_k(slots);
-
-    // ---- tile maxima ----
-    const int tile0 = (it * NW + wave) * 16;
+    // The maxima below are taken by instructions that the compiler does not look
+    // into, so it puts no wait states between them and the MFMAs.
+    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(sc[0]), "+v"(sc[1]));
     if constexpr (kGeneral) {
 #pragma unroll
       for (int i = 0; i < kRG; ++i)
@@ -272,140 +393,159 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
         for (int j = 0; j < 4; ++j)
           sc[i][j] = tile0 + 4 * grp + j < count[i] ? sc[i][j] : kNegBig;
     }
+    float mx[kRG];
 #pragma unroll
-    for (int i = 0; i < kRG; ++i) {
-      float mx = max3_raw(sc[i][0], sc[i][1], raw_max(sc[i][2], sc[i][3]));
-      float a, b;
-      pair16(mx, a, b);
-      mx = raw_max(a, b);
-      pair32(mx, a, b);
-      mx = raw_max(a, b);
-      if (grp == 0) tmax[16 * i + r16][wave] = mx;
-    }
+    for (int i = 0; i < kRG; ++i)
+      mx[i] = max3_raw(sc[i][0], sc[i][1], raw_max(sc[i][2], sc[i][3]));
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) mx[i] = groups_max(mx[i]);
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) *pub_max[i] = mx[i];
+    // Also the point from which the K tile may be refilled: its reads are done.
     lds_barrier();
 
-    // ---- the iteration's corrections, this tile's weights ----
-    float total[kRG];
-    bool big = false;
+    // ---- the iteration's corrections and this tile's weights; the K loads of
+    // the next iteration go out along the way ----
+    const char* kb = k_base(slots_next);
+    slots = slots_next;
+    slots_next = tile_slots(min(it + 2, n_it - 1));
+    int issued = 0;
+    auto k_load = [&]() {
+      if (issued < kKLoads / 4) stage_k4(issued++, kb);
+    };
+    // Group grp of 16 lanes handles tile grp; the running maximum before it comes
+    // from the other groups' maxima.
+    float tm[kRG];
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) tm[i] = tmax[16 * i + r16][grp];
+    k_load();
+    float m_t[kRG], c[kRG];
 #pragma unroll
     for (int i = 0; i < kRG; ++i) {
-      // Group grp of 16 lanes handles tiles kTPG * grp ..; the running maximum
-      // before them comes from the other groups' maxima.
-      float tm[kTPG];
-      if constexpr (kTPG == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(&tmax[16 * i + r16][2 * grp]);
-        tm[0] = v.x;
-        tm[1] = v.y;
-      } else {
-        tm[0] = tmax[16 * i + r16][grp];
-      }
-      const float gmax = kTPG == 2 ? raw_max(tm[0], tm[kTPG - 1]) : tm[0];
       float lo16, hi16, lo32, hi32;
-      pair16(gmax, lo16, hi16);
-      const float pmax = raw_max(lo16, hi16);
-      pair32(pmax, lo32, hi32);
-      const float m_end = max3_raw(m[i], lo32, hi32);
-      const float e1 = (grp & 1) ? lo16 : kNegBig;
-      const float e2 = (grp & 2) ? lo32 : kNegBig;
-      float mb = max3_raw(m[i], e1, e2);  // before the group's first tile
-      float own_total = 1.0f, own_after = 1.0f, m_sel = mb;
+      pair16(tm[i], lo16, hi16);
+      pair32(raw_max(lo16, hi16), lo32, hi32);
+      const float mb = max3_raw(m[i], (grp & 1) ? lo16 : kNegBig, (grp & 2) ? lo32 : kNegBig);
+      m[i] = max3_raw(m[i], lo32, hi32);
+      m_t[i] = raw_max(mb, tm[i]);
+      c[i] = fexp_fused_u(__builtin_fmaf(kExpA, mb - m_t[i], kExpBias));
+      if constexpr (kGeneral) c[i] = (it * kNW + grp) * 16 < count[i] ? c[i] : 1.0f;
+    }
+    // total: the product of all corrections; after: of those later than this
+    // wave's tile; m_w: the running maximum after it (held by group `wave`).
+    float total[kRG], after[kRG], m_w[kRG];
 #pragma unroll
-      for (int t = 0; t < kTPG; ++t) {
-        const int tile = kTPG * grp + t;  // of the iteration
-        const float mn = raw_max(mb, tm[t]);
-        float c = fexp_fused_u(__builtin_fmaf(kExpA, mb - mn, kExpBias));
-        if constexpr (kGeneral) c = (it * NW + tile) * 16 < count[i] ? c : 1.0f;
-        own_total *= c;
-        own_after *= tile > wave ? c : 1.0f;
-        if (t == 0 || (wave % kTPG) == t) m_sel = mn;
-        mb = mn;
-      }
-      total[i] = groups_mul(own_total);
-      const float after = groups_mul(own_after);
-      // m after tile `wave`: held by group wave / kTPG.
-      pair16(m_sel, lo16, hi16);
-      m_sel = (wave / kTPG) & 1 ? hi16 : lo16;
-      pair32(m_sel, lo32, hi32);
-      const float m_w = (wave / kTPG) & 2 ? hi32 : lo32;
-      m[i] = m_end;
-
-      const float t_arg = __builtin_fmaf(-kExpA, m_w, kExpBias);
-      float e[4];
+    for (int i = 0; i < kRG; ++i) {
+      total[i] = groups_mul(c[i]);
+      after[i] = groups_mul(grp > wave ? c[i] : 1.0f);
+      float lo, hi;
+      pair16(m_t[i], lo, hi);
+      pair32(wave & 1 ? hi : lo, lo, hi);
+      m_w[i] = wave & 2 ? hi : lo;
+    }
+    k_load();
+    float e[kRG][4], ts[kRG];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) e[j] = fexp_fused_u(__builtin_fmaf(kExpA, sc[i][j], t_arg));
+    for (int i = 0; i < kRG; ++i) {
+      const float t_arg = __builtin_fmaf(-kExpA, m_w[i], kExpBias);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) e[i][j] = fexp_fused_u(__builtin_fmaf(kExpA, sc[i][j], t_arg));
       if constexpr (kGeneral) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) e[j] = tile0 + 4 * grp + j < count[i] ? e[j] : 0.0f;
+        for (int j = 0; j < 4; ++j) e[i][j] = tile0 + 4 * grp + j < count[i] ? e[i][j] : 0.0f;
       }
-      const float ts = groups_add((e[0] + e[1]) + (e[2] + e[3])) * after;
-      big = big || ts > kLoShare * __builtin_fmaf(l[i], total[i], ts);
-      // acc = acc_stored * S: the corrections go into S, the weights are
-      // divided by it; below 2^-64 the accumulators take it over.
-      float S_new = S[i] * total[i];
-      if (__builtin_amdgcn_ballot_w64(S_new < 0x1p-64f) != 0) {  // wave-uniform
-#pragma unroll
-        for (int b = 0; b < kDB; ++b) acc[b][i] = acc[b][i] * S_new;
-        S_new = 1.0f;
-      }
-      S[i] = S_new;
-      const float fs = after * __builtin_amdgcn_rcpf(S_new);
-      typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-      float p[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) p[j] = e[j] * fs;
-      bf16x4_t h, lw;
-#pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        const bf16x2_t hb = __builtin_convertvector(f32x2_t{p[j], p[j + 1]}, bf16x2_t);
-        h[j] = hb[0];
-        h[j + 1] = hb[1];
-        const bf16x2_t lb = __builtin_convertvector(
-            f32x2_t{p[j] - static_cast<float>(hb[0]), p[j + 1] - static_cast<float>(hb[1])},
-            bf16x2_t);
-        lw[j] = lb[0];
-        lw[j + 1] = lb[1];
-      }
-      const int po = (16 * i + r16) * kPRow +
-                     16 * ((2 * wave + (grp >> 1)) ^ p_swz_row) + 8 * (grp & 1);
-      *reinterpret_cast<uint2*>(phi + po) = __builtin_bit_cast(uint2, h);
-      *reinterpret_cast<uint2*>(plo + po) = __builtin_bit_cast(uint2, lw);
-      if (grp == 0) tsum[16 * i + r16][wave] = ts;
+      k_load();
     }
-    const bool any_big = __builtin_amdgcn_ballot_w64(big) != 0;
-    if (lane == 0) big_flag[wave] = any_big ? 1 : 0;
-    lds_barrier();
-
-    // ---- l, and P.V over this wave's dims ----
+    bool big = false;
+    float S_new[kRG];
 #pragma unroll
     for (int i = 0; i < kRG; ++i) {
-      float sum = 0.0f;
+      ts[i] = groups_add((e[i][0] + e[i][1]) + (e[i][2] + e[i][3])) * after[i];
+      big = big || ts[i] > kLoShare * __builtin_fmaf(l[i], total[i], ts[i]);
+      S_new[i] = S[i] * total[i];
+    }
+    // acc = acc_stored * S: the corrections go into S, the weights are divided
+    // by it; below 2^-64 the accumulators take it over.
+    bool small = false;
 #pragma unroll
-      for (int t = 0; t < NW; t += 4) {
-        const float4 v = *reinterpret_cast<const float4*>(&tsum[16 * i + r16][t]);
-        sum += (v.x + v.y) + (v.z + v.w);
+    for (int i = 0; i < kRG; ++i) small = small || S_new[i] < 0x1p-64f;
+    if (__builtin_amdgcn_ballot_w64(small) != 0) {  // wave-uniform
+#pragma unroll
+      for (int i = 0; i < kRG; ++i) {
+#pragma unroll
+        for (int b = 0; b < kDB; ++b) acc[b][i] = acc[b][i] * S_new[i];
+        S_new[i] = 1.0f;
       }
-      l[i] = __builtin_fmaf(l[i], total[i], sum);
     }
-    int any = 0;
+    const bool any_big = __builtin_amdgcn_ballot_w64(big) != 0;  // wave-uniform
+    float p[kRG][4];
+    bf16x4_t h[kRG];
 #pragma unroll
-    for (int t = 0; t < NW; t += 4) {
-      const int4 v = *reinterpret_cast<const int4*>(&big_flag[t]);
-      any |= (v.x | v.y) | (v.z | v.w);
+    for (int i = 0; i < kRG; ++i) {
+      S[i] = S_new[i];
+      const float fs = after[i] * __builtin_amdgcn_rcpf(S_new[i]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[i][j] = e[i][j] * fs;
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const bf16x2_t hb = __builtin_convertvector(f32x2_t{p[i][j], p[i][j + 1]}, bf16x2_t);
+        h[i][j] = hb[0];
+        h[i][j + 1] = hb[1];
+      }
+      *reinterpret_cast<uint2*>(phi + p_write[i]) = __builtin_bit_cast(uint2, h[i]);
+      *pub_sum[i] = ts[i];
     }
-    __builtin_amdgcn_s_waitcnt(vmcnt_only(kKLoads + 1));  // V landed
-    bf16x8_t vf[kPS][kDB];
+#pragma unroll
+    for (int i = 0; i < kKLoads / 4; ++i) k_load();
+    // The lo parts p - hi: zeros when no row draws more than kLoShare of its l
+    // from the tile (its step's other tile may have some).
+    uint2 lo_bits[kRG];
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) lo_bits[i] = make_uint2(0u, 0u);
+    if (any_big) {
+#pragma unroll
+      for (int i = 0; i < kRG; ++i) {
+        bf16x4_t lw;
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+          const bf16x2_t lb = __builtin_convertvector(
+              f32x2_t{p[i][j] - static_cast<float>(h[i][j]),
+                      p[i][j + 1] - static_cast<float>(h[i][j + 1])},
+              bf16x2_t);
+          lw[j] = lb[0];
+          lw[j + 1] = lb[1];
+        }
+        lo_bits[i] = __builtin_bit_cast(uint2, lw);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) *reinterpret_cast<uint2*>(plo + p_write[i]) = lo_bits[i];
+    big_flag[wave] = any_big ? 1 : 0;
+    lds_barrier();
+
+    // ---- P.V over this wave's dims, and l ----
+    int flags[kNW];
+#pragma unroll
+    for (int t = 0; t < kNW; t += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(&big_flag[t]);
+      flags[t] = v.x;
+      flags[t + 1] = v.y;
+      flags[t + 2] = v.z;
+      flags[t + 3] = v.w;
+    }
+    wait_loads<kKLoads>();  // V landed (the K loads came after it)
+    bf16x8_t vf[kPS][kDB], ph[kPS][kRG], pl[kPS][kRG];
 #pragma unroll
     for (int s = 0; s < kPS; ++s) {
-      bf16x8_t ph[kRG];
 #pragma unroll
       for (int i = 0; i < kRG; ++i)
-        ph[i] = *reinterpret_cast<const bf16x8_t*>(phi + (16 * i + r16) * kPRow +
-                                                   16 * ((4 * s + grp) ^ p_swz_row));
+        ph[s][i] = *reinterpret_cast<const bf16x8_t*>(phi + (16 * i + r16) * kPRow +
+                                                      16 * ((4 * s + grp) ^ p_swz_row));
 #pragma unroll
       for (int b = 0; b < kDB; ++b) {
-        const int ka = 32 * s + vkey, kb = ka + 4;
+        const int ka = 32 * s + vkey, kb2 = ka + 4;
         const uint8_t* pa = vw + ka * kVB + 32 * (b ^ v_swz(ka)) + 8 * (r16 & 3);
-        const uint8_t* pb = vw + kb * kVB + 32 * (b ^ v_swz(kb)) + 8 * (r16 & 3);
+        const uint8_t* pb = vw + kb2 * kVB + 32 * (b ^ v_swz(kb2)) + 8 * (r16 & 3);
         const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)pa);
         const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)pb);
         vf[s][b] = __builtin_bit_cast(bf16x8_t,
@@ -415,35 +555,42 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
       for (int b = 0; b < kDB; ++b)
 #pragma unroll
         for (int i = 0; i < kRG; ++i)
-          acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s][b], ph[i], acc[b][i], 0, 0, 0);
+          acc[b][i] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s][b], ph[s][i], acc[b][i], 0, 0, 0);
     }
-    // The slice is in registers: refill it.
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    stage_v(general, itn, slots);
-    // The lo parts, on the same V fragments, when some row of the block draws
-    // more than kLoShare of its running l from a tile of the iteration.
-    if (__builtin_amdgcn_readfirstlane(any) != 0) {
+    // The lo parts on the same V fragments, for the steps with a flagged tile;
+    // read in any case: a read inside the branch would be waited for on its own.
 #pragma unroll
-      for (int s = 0; s < kPS; ++s) {
-        bf16x8_t pl[kRG];
+    for (int s = 0; s < kPS; ++s)
 #pragma unroll
-        for (int i = 0; i < kRG; ++i)
-          pl[i] = *reinterpret_cast<const bf16x8_t*>(plo + (16 * i + r16) * kPRow +
-                                                     16 * ((4 * s + grp) ^ p_swz_row));
+      for (int i = 0; i < kRG; ++i)
+        pl[s][i] = *reinterpret_cast<const bf16x8_t*>(plo + (16 * i + r16) * kPRow +
+                                                      16 * ((4 * s + grp) ^ p_swz_row));
+#pragma unroll
+    for (int i = 0; i < kRG; ++i) {
+      float sum = 0.0f;
+#pragma unroll
+      for (int t = 0; t < kNW; t += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(&tsum[16 * i + r16][t]);
+        sum += (v.x + v.y) + (v.z + v.w);
+      }
+      l[i] = __builtin_fmaf(l[i], total[i], sum);
+    }
+#pragma unroll
+    for (int s = 0; s < kPS; ++s)
+      if (__builtin_amdgcn_readfirstlane(flags[2 * s] | flags[2 * s + 1]) != 0) {
 #pragma unroll
         for (int b = 0; b < kDB; ++b)
 #pragma unroll
           for (int i = 0; i < kRG; ++i)
             acc[b][i] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s][b], pl[i], acc[b][i], 0, 0, 0);
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[s][b], pl[s][i], acc[b][i], 0, 0, 0);
       }
-    }
-    slots = slots_after;
+    // The slice is in registers: the next iteration may refill it.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
-  // Iterations below it_full and the ones they stage lie below every row's
-  // last key.
-  const int it_full = min_count / kKI - 1;
+  // The keys of iterations below it_full are valid for every row.
+  const int it_full = min_count / kKI;
   int it = 0;
   for (; it < it_full; ++it) iteration(std::false_type{}, it);
   for (; it < n_it; ++it) iteration(std::true_type{}, it);
@@ -472,9 +619,437 @@ void prefill_narrow_kernel(const int32_t* __restrict__ image, const uint16_t* __
   }
 }
 
+constexpr int kNKeys = 32 * kNW;   // keys per iteration
+constexpr int kNTiles = 2 * kNW;   // 16-key tiles per iteration
+
+template <int D, int G>
+__global__ __launch_bounds__(64 * kNW) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void prefill_narrow_pairs_kernel(const int32_t* __restrict__ image, const uint16_t* __restrict__ q,
+                           const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+                           uint16_t* __restrict__ out, int num_q, int num_kv,
+                           int64_t kv_stride, int shift, int row_mask) {
+  constexpr int kTok = kNRows / G;              // tokens of a block
+  constexpr int kKS = D / 16;                   // score MFMA steps
+  constexpr int kRowB = 2 * D;                  // bytes of a K row
+  constexpr int kDW = D / kNW;              // output dims of a wave
+  constexpr int kDB = kDW / 32;                 // 32-dim blocks of it
+  constexpr int kVB = 2 * kDW;                  // bytes of a V row slice in LDS
+  constexpr int kKRows = 1024 / kRowB;          // K rows per 1 KiB load
+  constexpr int kKLoads = 32 / kKRows;          // loads of a wave's 32 K rows
+  constexpr int kLPK = kVB / 16;                // lanes per V row slice
+  constexpr int kKPL = 64 / kLPK;               // V rows per load
+  constexpr int kVLoads = kNKeys / kKPL;
+  static_assert(kVLoads == kKS && kKLoads == kKS, "one V load per score step");
+
+  __shared__ __align__(16) uint8_t kbuf[kNKeys * kRowB];
+  __shared__ __align__(16) uint8_t vbuf[kNW * kNKeys * kVB];
+  __shared__ __align__(16) uint4 phi[kNTiles][64];
+  __shared__ __align__(16) uint4 plo[kNTiles][64];
+  __shared__ __align__(16) float tmax[kNRows][kNTiles];
+  __shared__ __align__(16) float tsum[kNRows][kNTiles];
+  __shared__ __align__(16) int32_t big_flag[kNTiles];
+
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 31;       // row of the block
+  const int half = lane >> 5;
+  const int g = blockIdx.x % num_kv;
+  const int rest = blockIdx.x / num_kv;
+  int qb, sub;
+  pick_sub_block<kTok>(image, rest, qb, sub);
+  if (qb < 0) return;  // block-uniform
+
+  const int32_t* blk = image + image[kHdrOffQBlocks] + qb * kQBlockWords;
+  const int run = blk[0];
+  const int t0 = blk[1] + sub * kTok;
+  const int ntok = min(kTok, blk[2] - sub * kTok);
+  const int32_t* rp = image + image[kHdrOffRuns] + run * 4;
+  const int pos0 = rp[1] + (t0 - rp[0]);  // first token's position
+  const int32_t* rows = image + image[kHdrOffRows] + rp[2];
+
+  const int min_count = pos0 + 1;         // keys below are valid for every row
+  const int count_max = pos0 + ntok;      // keys the block needs
+  const int last_tile = (count_max - 1) >> 4;
+  const int n_it = (count_max + kNKeys - 1) / kNKeys;
+
+  // Row r: token r / G, q head g * G + r % G.  Rows past the last token repeat
+  // it and are not stored.
+  const int tl = min(r / G, ntok - 1);
+  const bool live = r / G < ntok;
+  const int count = min_count + tl;
+  const int64_t q_row = static_cast<int64_t>(t0 + tl) * num_q + g * G + r % G;
+  bf16x8_t qf[kKS];
+  {
+    const uint16_t* qr = q + q_row * D + 8 * half;
+#pragma unroll
+    for (int s = 0; s < kKS; ++s) qf[s] = *reinterpret_cast<const bf16x8_t*>(qr + 16 * s);
+  }
+
+  // ---- staging ----
+  // The wave's 32 K rows: row k's 16-byte chunk c at c ^ (k % 16), so the rows
+  // of a fragment read lie in different bank groups.  V slice: the 32-byte
+  // unit u of key k at u ^ f(k), f spreading the 16 keys that a transposing
+  // read touches over the units of 256 bytes.
+  uint8_t* kw = kbuf + wave * 32 * kRowB;
+  uint8_t* vw = vbuf + wave * kNKeys * kVB;
+  const int64_t row_bytes = kv_stride * 2;
+  const uint32_t rb32 = static_cast<uint32_t>(row_bytes);
+  const char* kg = reinterpret_cast<const char*>(kc + static_cast<int64_t>(g) * D);
+  const char* vg = reinterpret_cast<const char*>(vc + static_cast<int64_t>(g) * D + wave * kDW);
+  auto v_swz = [](int key) -> int {
+    if constexpr (kVB == 128) return ((key >> 1) & 1) | (((key >> 2) & 1) << 1);
+    else return key & 7;
+  };
+  // First cache rows of the tiles of iteration it, tile t in lane t (pages hold
+  // whole tiles: page_len >= 16); tiles past the last one repeat it.  Loaded an
+  // iteration before the staging that uses them.
+  auto tile_slots = [&](int it) -> int {
+    const int key = 16 * min(it * kNTiles + (lane & (kNTiles - 1)), last_tile);
+    return rows[key >> shift] + (key & row_mask);
+  };
+  auto slot_of = [&](int sl, int t) -> int64_t { return __builtin_amdgcn_readlane(sl, t); };
+  // A K tile is 16 rows in kTL loads, 4 at a time; row kKRows * i + k_lrow of
+  // load i, its chunk ^ the row.  Rows past the block's last key are other rows
+  // of its page; their scores are masked.
+  constexpr int kTL = kKLoads / 2;
+  const int k_lrow = lane / (64 / kKRows);
+  uint32_t k_off[kTL];
+#pragma unroll
+  for (int i = 0; i < kTL; ++i) {
+    const int row = kKRows * i + k_lrow;
+    k_off[i] = static_cast<uint32_t>(row) * rb32 +
+               16u * static_cast<uint32_t>((lane % (64 / kKRows)) ^ row) + 1024u * (3 - i % 4);
+  }
+  auto stage_k4 = [&](int i4, const char* kb) {  // loads 4 * i4 .. of the wave's two tiles
+    const int i = 4 * i4 % kTL;
+    load_lds4(kb - 3072, k_off[i], k_off[i + 1], k_off[i + 2], k_off[i + 3], kw + i4 * 4096);
+  };
+  auto k_base = [&](int sl, int t) { return kg + slot_of(sl, 2 * wave + t) * row_bytes; };
+  // Tile t of the wave's V slice of iteration it, 16 rows in kVT loads.  tail:
+  // the iteration may reach past the last key; keys past it repeat a valid row
+  // (their weights are 0, and its values finite).
+  constexpr int kVT = 16 / kKPL;
+  static_assert(kVT == 2 || kVT == 4, "V loads of a tile");
+  const int v_lrow = lane / kLPK;
+  uint32_t v_chunk[kVT], v_off[kVT];
+#pragma unroll
+  for (int i = 0; i < kVT; ++i) {
+    const int row = kKPL * i + v_lrow;
+    v_chunk[i] = 16u * static_cast<uint32_t>((lane % kLPK) ^ (2 * v_swz(row))) + 1024u * (kVT - 1 - i);
+    v_off[i] = static_cast<uint32_t>(row) * rb32 + v_chunk[i];
+  }
+  auto stage_v = [&](auto tail, int t, int it, int sl) {
+    const char* vb = vg + slot_of(sl, t) * row_bytes - 1024 * (kVT - 1);
+    uint32_t off[kVT];
+#pragma unroll
+    for (int i = 0; i < kVT; ++i) {
+      off[i] = v_off[i];
+      if constexpr (tail.value) {
+        const int last = count_max - 1 - 16 * min(it * kNTiles + t, last_tile);
+        off[i] = static_cast<uint32_t>(min(kKPL * i + v_lrow, last)) * rb32 + v_chunk[i];
+      }
+    }
+    if constexpr (kVT == 2) load_lds2(vb, off[0], off[1], vw + t * 2048);
+    else load_lds4(vb, off[0], off[1], off[2], off[3], vw + t * 4096);
+  };
+
+  // ---- per-row state, the same in both lanes of a row ----
+  float m = kNegBig, l = 0.0f, S = 1.0f;
+  f32x16_t acc[kDB];
+#pragma unroll
+  for (int b = 0; b < kDB; ++b)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[b][v] = 0.0f;
+
+  int slots = tile_slots(0);                      // of the iteration at hand
+  int slots_next = tile_slots(min(1, n_it - 1));  // and of the one after it
+#pragma unroll
+  for (int i = 0; i < kKLoads / 4; ++i) stage_k4(i, k_base(slots, 4 * i / kTL));
+
+  const int k_read = r * kRowB + 16 * ((r & 15) ^ half);  // fragment s at k_read ^ 32 s
+  // Transposing read of dim block b of a tile: lane j of 16-lane group q
+  // addresses key 4 * half + j / 4 (+ 8 for the second read), dims
+  // 16 * (q % 2) + 4 * (j % 4) .. +3, and gets the four keys of dim
+  // 16 * (q % 2) + j: the k order of the lane's own P values.
+  const int j16 = lane & 15;
+  const int vkey = 4 * half + (j16 >> 2);
+  const int vunit = (lane >> 4) & 1;
+
+  // One iteration.  general: some rows may end inside it.
+  auto iteration = [&](auto general, int it) {
+    constexpr bool kGeneral = general.value;
+    const int key0 = it * kNKeys + 32 * wave;  // of the wave's two tiles
+    // ---- scores, with the V loads of the iteration between the MFMAs (the
+    // slice was read by the last P.V) ----
+    f32x16_t sc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
+    wait_loads<0>();  // K landed
+    bf16x8_t kf[kKS];
+#pragma unroll
+    for (int s = 0; s < kKS; ++s)
+      kf[s] = *reinterpret_cast<const bf16x8_t*>(kw + (k_read ^ (32 * s)));
+#pragma unroll
+    for (int s = 0; s < kKS; ++s) {
+      if (s % (kKS / kNTiles) == 0) stage_v(general, s / (kKS / kNTiles), it, slots);
+      sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], qf[s], sc, 0, 0, 0);
+    }
+    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(sc));
+    // Value 8 u + i of a lane is key 16 u + 8 (i / 4) + 4 half + i % 4.
+    if constexpr (kGeneral) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        sc[v] = key0 + 8 * (v >> 2) + 4 * half + (v & 3) < count ? sc[v] : kNegBig;
+    }
+    float mx[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float sv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sv[i] = sc[8 * u + i];
+      mx[u] = max8(sv);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float a, b;
+      pair32(mx[u], a, b);
+      mx[u] = raw_max(a, b);
+    }
+    tmax[r][2 * wave + half] = half ? mx[1] : mx[0];
+    // Also the point from which the K rows may be refilled: their reads are done.
+    lds_barrier();
+
+    // ---- the iteration's corrections and these tiles' weights; the K loads of
+    // the next iteration go out along the way ----
+    const char* kb0 = k_base(slots_next, 0);
+    const char* kb1 = k_base(slots_next, 1);
+    slots = slots_next;
+    slots_next = tile_slots(min(it + 2, n_it - 1));
+    int issued = 0;
+    auto k_load = [&]() {
+      if (issued < kKLoads / 4) {
+        stage_k4(issued, 4 * issued < kTL ? kb0 : kb1);
+        ++issued;
+      }
+    };
+    // Half h of the lanes handles tiles 4 h .. 4 h + 3; the running maximum
+    // before tile 4 comes from the other half's maxima.
+    const float4 tm4 = *reinterpret_cast<const float4*>(&tmax[r][4 * half]);
+    const float tm[4] = {tm4.x, tm4.y, tm4.z, tm4.w};
+    k_load();
+    float mn[4], c[4], lo, hi;
+    pair32(raw_max(max3_raw(tm[0], tm[1], tm[2]), tm[3]), lo, hi);
+    {
+      float mb = half ? raw_max(m, lo) : m;
+      m = max3_raw(m, lo, hi);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        mn[t] = raw_max(mb, tm[t]);
+        c[t] = fexp_fused_u(__builtin_fmaf(kExpA, mb - mn[t], kExpBias));
+        if constexpr (kGeneral)
+          c[t] = (it * kNTiles + 4 * half + t) * 16 < count ? c[t] : 1.0f;
+        mb = mn[t];
+      }
+    }
+    // Of this wave's tiles a = 2 wave and b = a + 1, both held by half wave / 2:
+    // the maxima after them, b's correction, and the product of the later ones.
+    const float own_total = (c[0] * c[1]) * (c[2] * c[3]);
+    const bool second = wave & 1;
+    float own_after = (second ? 1.0f : c[2]) * (second ? 1.0f : c[3]);
+    own_after = (wave >> 1) == half ? own_after : ((wave >> 1) < half ? own_total : 1.0f);
+    pair32(own_total, lo, hi);
+    const float total = lo * hi;
+    pair32(own_after, lo, hi);
+    const float after_b = lo * hi;
+    pair32(second ? mn[2] : mn[0], lo, hi);
+    const float m_a = wave >> 1 ? hi : lo;
+    pair32(second ? mn[3] : mn[1], lo, hi);
+    const float m_b = wave >> 1 ? hi : lo;
+    pair32(second ? c[3] : c[1], lo, hi);
+    const float after_a = after_b * (wave >> 1 ? hi : lo);
+    const float after[2] = {after_a, after_b};
+    const float ta[2] = {__builtin_fmaf(-kExpA, m_a, kExpBias), __builtin_fmaf(-kExpA, m_b, kExpBias)};
+    float e[2][8], ts[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        e[u][i] = fexp_fused_u(__builtin_fmaf(kExpA, sc[8 * u + i], ta[u]));
+        if constexpr (kGeneral)
+          e[u][i] = key0 + 16 * u + 8 * (i >> 2) + 4 * half + (i & 3) < count ? e[u][i] : 0.0f;
+      }
+      k_load();
+      ts[u] = ((e[u][0] + e[u][1]) + (e[u][2] + e[u][3])) + ((e[u][4] + e[u][5]) + (e[u][6] + e[u][7]));
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      pair32(ts[u], lo, hi);
+      ts[u] = (lo + hi) * after[u];
+    }
+    tsum[r][2 * wave + half] = half ? ts[1] : ts[0];
+    // acc = acc_stored * S: the corrections go into S, the weights are divided
+    // by it; below 2^-64 the accumulators take it over.
+    float S_new = S * total;
+    if (__builtin_amdgcn_ballot_w64(S_new < 0x1p-64f) != 0) {  // wave-uniform
+#pragma unroll
+      for (int b = 0; b < kDB; ++b) acc[b] = acc[b] * S_new;
+      S_new = 1.0f;
+    }
+    S = S_new;
+    const float inv_s = __builtin_amdgcn_rcpf(S_new);
+    // P in bf16 hi parts; a tile also gets its lo parts p - hi when it draws
+    // more than kLoShare of some row's l.
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const float fs = after[u] * inv_s;
+      float p[8];
+      bf16x8_t h;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = e[u][i] * fs;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        const bf16x2_t hb = __builtin_convertvector(f32x2_t{p[i], p[i + 1]}, bf16x2_t);
+        h[i] = hb[0];
+        h[i + 1] = hb[1];
+      }
+      phi[2 * wave + u][lane] = __builtin_bit_cast(uint4, h);
+      const bool big = __builtin_amdgcn_ballot_w64(
+                           ts[u] > kLoShare * __builtin_fmaf(l, total, ts[u])) != 0;
+      if (big) {  // wave-uniform
+        bf16x8_t w;
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+          const bf16x2_t lb = __builtin_convertvector(
+              f32x2_t{p[i] - static_cast<float>(h[i]), p[i + 1] - static_cast<float>(h[i + 1])},
+              bf16x2_t);
+          w[i] = lb[0];
+          w[i + 1] = lb[1];
+        }
+        plo[2 * wave + u][lane] = __builtin_bit_cast(uint4, w);
+      }
+      big_flag[2 * wave + u] = big ? 1 : 0;
+      k_load();
+    }
+#pragma unroll
+    for (int i = 0; i < kKLoads / 4; ++i) k_load();
+    lds_barrier();
+
+    // ---- P.V over this wave's dims, and l ----
+    int flags[kNTiles];
+#pragma unroll
+    for (int t = 0; t < kNTiles; t += 4) {
+      const int4 v = *reinterpret_cast<const int4*>(&big_flag[t]);
+      flags[t] = v.x;
+      flags[t + 1] = v.y;
+      flags[t + 2] = v.z;
+      flags[t + 3] = v.w;
+    }
+    // V landed: the K loads issued after it may be outstanding.
+    wait_loads<kKLoads>();
+    bf16x8_t vf[kNTiles][kDB];
+    bf16x8_t ph[kNTiles];
+#pragma unroll
+    for (int t = 0; t < kNTiles; ++t) {
+      ph[t] = __builtin_bit_cast(bf16x8_t, phi[t][lane]);
+#pragma unroll
+      for (int b = 0; b < kDB; ++b) {
+        const int ka = 16 * t + vkey, kb = ka + 8;
+        const int u = 2 * b + vunit;
+        const uint8_t* pa = vw + ka * kVB + 32 * (u ^ v_swz(ka)) + 8 * (j16 & 3);
+        const uint8_t* pb = vw + kb * kVB + 32 * (u ^ v_swz(kb)) + 8 * (j16 & 3);
+        const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)pa);
+        const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)pb);
+        vf[t][b] = __builtin_bit_cast(bf16x8_t,
+                                      __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < kNTiles; ++t)
+#pragma unroll
+      for (int b = 0; b < kDB; ++b)
+        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][b], ph[t], acc[b], 0, 0, 0);
+    // Read whether or not the tile has lo parts: a read inside the branch
+    // would be waited for on its own.
+    bf16x8_t pl[kNTiles];
+#pragma unroll
+    for (int t = 0; t < kNTiles; ++t) pl[t] = __builtin_bit_cast(bf16x8_t, plo[t][lane]);
+    {
+      const float4 v0 = *reinterpret_cast<const float4*>(&tsum[r][0]);
+      const float4 v1 = *reinterpret_cast<const float4*>(&tsum[r][4]);
+      l = __builtin_fmaf(l, total, ((v0.x + v0.y) + (v0.z + v0.w)) + ((v1.x + v1.y) + (v1.z + v1.w)));
+    }
+#pragma unroll
+    for (int t = 0; t < kNTiles; ++t)
+      if (__builtin_amdgcn_readfirstlane(flags[t]) != 0) {
+#pragma unroll
+        for (int b = 0; b < kDB; ++b)
+          acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[t][b], pl[t], acc[b], 0, 0, 0);
+      }
+    // The slice is in registers: the next iteration may refill it.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  // The keys of iterations below it_full are valid for every row.
+  const int it_full = min_count / kNKeys;
+  int it = 0;
+  for (; it < it_full; ++it) iteration(std::false_type{}, it);
+  for (; it < n_it; ++it) iteration(std::true_type{}, it);
+  // No load may still be on its way into LDS when the workgroup ends.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  // ---- one-segment merge and bf16 store (PrefillMergeKernel) ----
+  // Value 4 j + i of block b is dim 32 b + 8 j + 4 half + i.
+  if (!live) return;
+  const float c0 = l > 0.0f ? fexp(0.0f) : 0.0f;
+  const float gl = l * c0;
+  const bool some = gl > 0.0f;
+  const float inv_l = some ? 1.0f / gl : 0.0f;
+  uint16_t* dst = out + q_row * D + wave * kDW + 4 * half;
+#pragma unroll
+  for (int b = 0; b < kDB; ++b)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float av = (acc[b][4 * j + i] * S) * c0;
+        w[i] = some ? f32_to_bf16_bits(av * inv_l) : 0u;
+      }
+      *reinterpret_cast<uint2*>(dst + 32 * b + 8 * j) =
+          make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+    }
+}
+
 }  // namespace
 
-hipError_t launch_prefill_narrow(const int32_t* image, int num_qblocks, const void* q,
+// Which kernel takes a full-attention token plan: 0 the query-block kernel, 1
+// tiles, 2 pairs.  A cost in us per 128 keys, from the measurements above: a
+// launch takes its 256 (or, tiles at head_dim 256, 512) blocks at a time.
+// live: blocks of 32 rows with tokens (an upper bound: every run may end in a
+// partial one).  The query-block kernels' later rounds overlap, so beyond one
+// round they cost their share of it.
+int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, int64_t num_kv,
+                        int head_dim, int64_t kv_stride, int page_shift) {
+  // Pages hold whole tiles, and a tile's row offsets fit 32 bits.
+  if (page_shift < 4 || kv_stride > (int64_t{1} << 25)) return 0;
+  auto rounds = [](int64_t blocks, int64_t at_once) {
+    return static_cast<double>((blocks + at_once - 1) / at_once);
+  };
+  auto block_cost = [](int64_t blocks, double one, double more) {
+    return blocks <= 256 ? one : (one > more * blocks / 256.0 ? one : more * blocks / 256.0);
+  };
+  if (head_dim == 256) {
+    const int64_t live = (seq_len + 15 * num_runs) / 16 * num_kv;
+    const double block = block_cost(num_qblocks * num_kv, 8.7, 6.5);
+    const double pairs = 2.45 * rounds(live, 256);
+    const double tiles = live <= 256 ? 3.2 : 4.3 * rounds(live, 512);
+    if (block <= pairs && block <= tiles) return 0;
+    return pairs <= tiles ? 2 : 1;
+  }
+  const int64_t live = (seq_len + 3 * num_runs) / 4 * num_kv;
+  return 5.05 * rounds(live, 256) < block_cost(4 * num_qblocks * num_kv, 11.5, 9.8) ? 1 : 0;
+}
+
+hipError_t launch_prefill_narrow(const int32_t* image, int kind, int num_qblocks, const void* q,
                                  const void* k, const void* v, void* output, int head_dim,
                                  int num_q, int num_kv, int64_t kv_stride, PagedGeom geom,
                                  hipStream_t stream) {
@@ -483,15 +1058,19 @@ hipError_t launch_prefill_narrow(const int32_t* image, int num_qblocks, const vo
   const auto* kp = static_cast<const uint16_t*>(k);
   const auto* vp = static_cast<const uint16_t*>(v);
   auto* op = static_cast<uint16_t*>(output);
-  if (head_dim == 256) {
-    hipLaunchKernelGGL((prefill_narrow_kernel<256, 2, 8>), dim3(num_qblocks * 4 * num_kv),
-                       dim3(512), 0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride,
-                       geom.shift, geom.row_mask);
-  } else {
-    hipLaunchKernelGGL((prefill_narrow_kernel<512, 8, 4>), dim3(num_qblocks * 16 * num_kv),
-                       dim3(256), 0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride,
-                       geom.shift, geom.row_mask);
-  }
+  const unsigned blocks = static_cast<unsigned>(num_qblocks) * static_cast<unsigned>(num_kv);
+  if (head_dim == 256 && kind == 2)
+    hipLaunchKernelGGL((prefill_narrow_pairs_kernel<256, 2>), dim3(blocks * 4), dim3(64 * kNW), 0,
+                       stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+                       geom.row_mask);
+  else if (head_dim == 256)
+    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<256, 2, 2>), dim3(blocks * 4), dim3(64 * kNW),
+                       0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+                       geom.row_mask);
+  else
+    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<512, 8, 1>), dim3(blocks * 16), dim3(64 * kNW),
+                       0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+                       geom.row_mask);
   return hipGetLastError();
 }
 
