@@ -309,6 +309,116 @@ __global__ __launch_bounds__(128) void append_vec_kernel(
   for (int i = threadIdx.x; i < (n_heads * head_dim) >> 3; i += blockDim.x) vd[i] = vs[i];
 }
 
+// The append with the norm at the compiled head sizes: 16 lanes hold a head row
+// in registers, lane j the bf16 pairs (32 p + 2 j, + 1), so the row is read once
+// and never again.  The sum of squares is group_inv_rms's, operation for
+// operation (its lane j sums the same pairs), and a rotation's partner, a
+// multiple of 32 elements away, is the lane's own.  Requires half and
+// pair_stride to be multiples of 32 (the launcher checks).
+//
+// Bound by HBM for many tokens and by its chain of loads for few; the kernel it
+// stands in for reads every element three times, two bytes at a time.  2,000
+// tokens of 16 q / 8 kv heads x 256: 31.6 -> 14.2 us (4.6 TB/s); one token 6.7
+// -> 3.5 us.
+template <int D>
+__global__ __launch_bounds__(16 * kGroupHeads) void append_norm_rows_kernel(
+    const int32_t* __restrict__ image, uint16_t* __restrict__ q,
+    const uint16_t* __restrict__ k_src, const uint16_t* __restrict__ v_src,
+    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
+    const uint16_t* __restrict__ q_w, const uint16_t* __restrict__ k_w,
+    const float* __restrict__ cos_table, const float* __restrict__ sin_table, int num_q,
+    int num_kv, int shift, int row_mask, int page_mask, int half, int pair_stride, float sqrt_n,
+    float n_eps) {
+  constexpr int kP = D / 32;  // pairs of a lane
+  constexpr int kPu = 8;      // the sum's accumulators: pair p goes to p % 8
+  const int tok = blockIdx.x;
+  const HeadGroup grp = head_group(blockIdx.y, num_q, num_kv);
+  const int j = threadIdx.x & 15;
+  const int h = grp.h0 + (threadIdx.x >> 4);
+  if (h >= grp.h1) return;  // uniform per 16-lane group
+  const int64_t row = static_cast<int64_t>(tok) * (grp.kind == 0 ? num_q : num_kv) + h;
+  const uint16_t* src = (grp.kind == 0 ? q : grp.kind == 1 ? k_src : v_src) + row * D;
+  uint32_t x[kP];
+#pragma unroll
+  for (int p = 0; p < kP; ++p) x[p] = reinterpret_cast<const uint32_t*>(src)[16 * p + j];
+  uint32_t w[kP];
+  if (grp.kind != 2) {
+    const auto* wp = reinterpret_cast<const uint32_t*>(grp.kind == 0 ? q_w : k_w);
+#pragma unroll
+    for (int p = 0; p < kP; ++p) w[p] = wp[16 * p + j];
+  }
+  const int run = image[image[kHdrOffTokRun] + tok];
+  const int32_t* rp = image + image[kHdrOffRuns] + run * 4;
+  const int pos = rp[1] + (tok - rp[0]);
+  uint16_t* dst;
+  if (grp.kind == 0) {
+    dst = q + row * D;
+  } else {
+    const int32_t* rows = image + image[kHdrOffRows] + rp[2];
+    const int64_t slot =
+        static_cast<int64_t>(rows[(pos >> shift) & page_mask]) + (pos & row_mask);
+    dst = (grp.kind == 1 ? k_cache : v_cache) + (slot * num_kv + h) * D;
+  }
+
+  float acc[kPu];
+#pragma unroll
+  for (int p = 0; p < kPu; ++p) acc[p] = 0.0f;
+#pragma unroll
+  for (int p = 0; p < kP; ++p) {
+    const float xe = bf16_lo(x[p]), xo = bf16_hi(x[p]);
+    float a = acc[p % kPu];
+    a = a + xo * xo;
+    a = a + xe * xe;
+    acc[p % kPu] = a;
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int p = 0; p < kPu; ++p) sum = sum + acc[p];
+  sum = tree16_sum(sum);
+  const float inv = sqrt_n / sqrtf(sum + n_eps);
+
+  uint32_t* out = reinterpret_cast<uint32_t*>(dst);
+  if (grp.kind == 2) {
+#pragma unroll
+    for (int p = 0; p < kP; ++p)
+      out[16 * p + j] = f32_to_bf16_bits(bf16_lo(x[p]) * inv) |
+                        (f32_to_bf16_bits(bf16_hi(x[p]) * inv) << 16);
+    return;
+  }
+  // The normalised row as the bf16 values the reference stores.
+  uint32_t y[kP];
+#pragma unroll
+  for (int p = 0; p < kP; ++p)
+    y[p] = f32_to_bf16_bits((bf16_lo(x[p]) * inv) * bf16_lo(w[p])) |
+           (f32_to_bf16_bits((bf16_hi(x[p]) * inv) * bf16_hi(w[p])) << 16);
+  const auto* cos_row = reinterpret_cast<const float2*>(cos_table + static_cast<int64_t>(pos) * half);
+  const auto* sin_row = reinterpret_cast<const float2*>(sin_table + static_cast<int64_t>(pos) * half);
+  const int hp = half >> 5, gap = pair_stride >> 5;
+  // The rotated pairs of the two compiled geometries (128 apart at D = 256, 256
+  // at D = 512, as many as half says); any other distance by selection.
+#pragma unroll
+  for (int p = 0; p < kP / 2; ++p) {
+    if (p >= hp) break;  // block-uniform
+    const float2 c = cos_row[16 * p + j], sn = sin_row[16 * p + j];
+    uint32_t other = y[p + kP / 2];
+    if (gap != kP / 2) {  // block-uniform
+#pragma unroll
+      for (int i = 0; i < kP; ++i) other = i == p + gap ? y[i] : other;
+    }
+    float lo0, hi0, lo1, hi1;
+    rotate(bf16_lo(y[p]), bf16_lo(other), c.x, sn.x, lo0, hi0);
+    rotate(bf16_hi(y[p]), bf16_hi(other), c.y, sn.y, lo1, hi1);
+    const uint32_t lo = f32_to_bf16_bits(lo0) | (f32_to_bf16_bits(lo1) << 16);
+    const uint32_t hi = f32_to_bf16_bits(hi0) | (f32_to_bf16_bits(hi1) << 16);
+    out[16 * p + j] = lo;
+    out[16 * (p + gap) + j] = hi;
+  }
+  // The unrotated rest.
+#pragma unroll
+  for (int p = 0; p < kP; ++p)
+    if (p >= hp && !(p >= gap && p < gap + hp)) out[16 * p + j] = y[p];
+}
+
 // In-place head RMS norm of q, k and v (one block per token and head group).
 __global__ __launch_bounds__(256) void rms_norm_qkv_kernel(
     uint16_t* __restrict__ q, uint16_t* __restrict__ k, uint16_t* __restrict__ v,
@@ -393,6 +503,29 @@ hipError_t launch_rms_rope_cache_write(const int32_t* image, int seq_len, void* 
                                        int pair_stride, int head_dim, float sqrt_n,
                                        float n_eps, hipStream_t stream) {
   if (seq_len <= 0) return hipSuccess;
+  const uintptr_t bases = reinterpret_cast<uintptr_t>(cos_table) |
+                          reinterpret_cast<uintptr_t>(sin_table);
+  const uintptr_t rows4 = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_src) |
+                          reinterpret_cast<uintptr_t>(v_src) |
+                          reinterpret_cast<uintptr_t>(k_cache) |
+                          reinterpret_cast<uintptr_t>(v_cache) |
+                          reinterpret_cast<uintptr_t>(q_w) | reinterpret_cast<uintptr_t>(k_w);
+  if ((head_dim == 256 || head_dim == 512) && half % 32 == 0 && pair_stride % 32 == 0 &&
+      half <= head_dim / 2 && (bases & 7) == 0 && (rows4 & 3) == 0) {
+    const dim3 grid(seq_len, num_head_groups(num_q, num_kv));
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(16 * kGroupHeads), 0, stream, image,
+                         static_cast<uint16_t*>(q), static_cast<const uint16_t*>(k_src),
+                         static_cast<const uint16_t*>(v_src), static_cast<uint16_t*>(k_cache),
+                         static_cast<uint16_t*>(v_cache), static_cast<const uint16_t*>(q_w),
+                         static_cast<const uint16_t*>(k_w), cos_table, sin_table, num_q, num_kv,
+                         geom.shift, geom.row_mask, geom.page_mask, half, pair_stride, sqrt_n,
+                         n_eps);
+      return hipGetLastError();
+    };
+    return head_dim == 256 ? run(append_norm_rows_kernel<256>)
+                           : run(append_norm_rows_kernel<512>);
+  }
   hipLaunchKernelGGL(append_kernel<true>, dim3(seq_len, num_head_groups(num_q, num_kv)),
                      dim3(256), 0, stream, image, static_cast<uint16_t*>(q),
                      static_cast<const uint16_t*>(k_src), static_cast<const uint16_t*>(v_src),

@@ -96,3 +96,11 @@ def test_norm_fused_into_append_bit_exact(kind, half, pair_stride):
     assert np.array_equal(from_dev(kcd, np.uint16), kc_r), "k cache"
     assert np.array_equal(from_dev(vcd, np.uint16), vc_r), "v cache"
     assert np.array_equal(from_dev(ksd, np.uint16), ks), "k_src is only read"
+
+
+@pytest.mark.parametrize("half,pair_stride", [(32, 160), (96, 160), (128, 128), (16, 128),
+                                              (8, 40)])
+def test_norm_append_rotation_geometries(half, pair_stride):
+    """The row kernel (half and pair_stride multiples of 32) at partner
+    distances other than half a head, and the element kernel for the rest."""
+    test_norm_fused_into_append_bit_exact(FULL, half, pair_stride)
