@@ -843,14 +843,68 @@ __global__ __launch_bounds__(256) void bq_block_quant_kernel(
   }
   if (lane == 0) x_sa[pair] = amax;
 }
+
+// The same at the attention's head sizes with everything 8- or 16-byte wide: a
+// wave holds a whole block in registers (4 or 8 values a lane), so the block is
+// read once.  Bound by HBM; 16,384 tokens x 16 heads x 256 (201 MB): 86 us for
+// the element kernel, 43 us here.
+template <int kBlock>
+__global__ __launch_bounds__(256) void bq_block_quant_vec_kernel(
+    const uint16_t* __restrict__ src, int8_t* __restrict__ x_i8, float* __restrict__ x_sa,
+    int64_t n_pairs) {
+  constexpr int kPer = kBlock / 64;  // values of a lane
+  typedef uint32_t words_t __attribute__((ext_vector_type(kPer / 2)));
+  const int lane = threadIdx.x & 63;
+  const int64_t pair = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (pair >= n_pairs) return;
+  const int64_t base = pair * kBlock + lane * kPer;
+  const words_t v = *reinterpret_cast<const words_t*>(src + base);
+  float x[kPer];
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kPer / 2; ++i) {
+    x[2 * i] = bf16_lo(v[i]);
+    x[2 * i + 1] = bf16_hi(v[i]);
+    amax = fmaxf(amax, fmaxf(fabsf(x[2 * i]), fabsf(x[2 * i + 1])));
+  }
+  amax = butterfly_all(amax, lane, [](float a, float o) { return fmaxf(a, o); });
+  const float inv = amax > 0.0f ? 127.0f / amax : 0.0f;
+  uint32_t out[kPer / 4];
+#pragma unroll
+  for (int i = 0; i < kPer / 4; ++i) {
+    out[i] = 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const float r = fminf(fmaxf(rintf(x[4 * i + b] * inv), -128.0f), 127.0f);
+      out[i] |= (static_cast<uint32_t>(static_cast<int32_t>(r)) & 0xFFu) << (8 * b);
+    }
+  }
+  if constexpr (kPer == 4)
+    *reinterpret_cast<uint32_t*>(x_i8 + base) = out[0];
+  else
+    *reinterpret_cast<uint2*>(x_i8 + base) = make_uint2(out[0], out[1]);
+  if (lane == 0) x_sa[pair] = amax;
+}
 }  // namespace
 
 hipError_t launch_bq_block_quant(const void* src, void* x_i8, float* x_sa, int64_t cols,
                                  int block, int64_t seq_len, hipStream_t stream) {
   if (seq_len <= 0) return hipSuccess;
   const int64_t pairs = static_cast<int64_t>(seq_len) * (cols / block);
-  hipLaunchKernelGGL(bq_block_quant_kernel, dim3(static_cast<unsigned>((pairs + 3) / 4)),
-                     dim3(256), 0, stream, static_cast<const uint16_t*>(src),
+  const dim3 grid(static_cast<unsigned>((pairs + 3) / 4));
+  const bool wide = (reinterpret_cast<uintptr_t>(src) & 15) == 0 &&
+                    (reinterpret_cast<uintptr_t>(x_i8) & 7) == 0;
+  if (wide && block == 256) {
+    hipLaunchKernelGGL(bq_block_quant_vec_kernel<256>, grid, dim3(256), 0, stream,
+                       static_cast<const uint16_t*>(src), static_cast<int8_t*>(x_i8), x_sa, pairs);
+    return hipGetLastError();
+  }
+  if (wide && block == 512) {
+    hipLaunchKernelGGL(bq_block_quant_vec_kernel<512>, grid, dim3(256), 0, stream,
+                       static_cast<const uint16_t*>(src), static_cast<int8_t*>(x_i8), x_sa, pairs);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(bq_block_quant_kernel, grid, dim3(256), 0, stream, static_cast<const uint16_t*>(src),
                      static_cast<int8_t*>(x_i8), x_sa, cols, block, pairs);
   return hipGetLastError();
 }
