@@ -78,6 +78,14 @@ def test_gemm_cols_tiles_bit_exact(seq, rows, cols):
     assert np.array_equal(got, oracle.f32_to_bf16((x @ w.T).ravel()).reshape(seq, rows))
 
 
+@pytest.mark.parametrize("seq,rows,cols", [(1, 16, 256), (1, 2816, 4096), (15, 48, 512),
+                                           (16, 2816, 8192), (7, 80, 1536), (17, 80, 4096)])
+def test_gemm_cols_few_tokens_bit_exact(seq, rows, cols):
+    """One to sixteen tokens (slices joined in the workgroup) and the first
+    size past them, 1 to 16 slices of 256 and 512."""
+    test_gemm_cols_integer_operands_bit_exact(seq, rows, cols)
+
+
 def test_gemm_cols_rejects_unsupported_shapes():
     from inferno_amd._lib import InfernoHipError
 
