@@ -30,7 +30,8 @@ OBJ_DIR = PKG.parent / "_build" / "obj"
 ARCH = "gfx950"
 
 SOURCES = ["api.hip", "attention.hip", "attention_wide.hip", "append.hip", "copy.hip", "bq.hip",
-           "prefill.hip", "prefill_narrow.hip", "prefill_sliding.hip", "prefill_wide.hip",
+           "prefill.hip", "prefill_narrow.hip", "prefill_pair.hip", "prefill_sliding.hip",
+           "prefill_wide.hip",
            "gemm.hip", "sparse.hip"]
 # Host-only C++ (page state, scheduler): built with the host compiler.
 HOST_SOURCES = ["host_state.cpp", "host_api.cpp"]

@@ -763,6 +763,14 @@ int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
   }
   if (route == PrefillRoute::kFull256) {
     // Prefill chunk of full attention: MFMA query blocks, finalised in-kernel.
+    if (ifr::prefill_pair_takes(kv_stride, static_cast<int>(pow2_shift(page_len)))) {
+      IFR_HIP(ifr::launch_prefill_pair(static_cast<const int32_t*>(image_dev),
+                                       static_cast<int>(info[14]), q, k_base, v_base, output,
+                                       static_cast<int>(num_q), static_cast<int>(num_kv),
+                                       kv_stride, g, as_stream(stream)),
+              "prefill_pair");
+      return ok();
+    }
     IFR_HIP(ifr::launch_prefill_full_mfma(static_cast<const int32_t*>(image_dev),
                                           static_cast<int>(info[14]), q, k_base, v_base,
                                           output, static_cast<int>(num_q),

@@ -49,7 +49,12 @@ hipError_t launch_prefill_full_mfma(const int32_t* image_dev, int num_qblocks,
                                     const void* v_base, void* output, int num_q,
                                     int num_kv, int64_t kv_stride, PagedGeom geom,
                                     hipStream_t stream);
-// The same over butterquant int8 KV (f32 scales per row and kv head).
+// The same plans over pages of 16 rows and more, two waves to a SIMD
+// (prefill_pair.hip); prefill_pair_takes: the layouts that it reads.
+bool prefill_pair_takes(int64_t kv_stride, int page_shift);
+hipError_t launch_prefill_pair(const int32_t* image, int num_qblocks, const void* q,
+                               const void* k, const void* v, void* output, int num_q, int num_kv,
+                               int64_t kv_stride, PagedGeom geom, hipStream_t stream);
 // Full-attention prefill of few rows: the kernel for a plan (0: none of these),
 // and its launch.
 int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, int64_t num_kv,
@@ -58,6 +63,7 @@ hipError_t launch_prefill_narrow(const int32_t* image, int kind, int num_qblocks
                                  const void* k, const void* v, void* output, int head_dim,
                                  int num_q, int num_kv, int64_t kv_stride, PagedGeom geom,
                                  hipStream_t stream);
+// prefill_full_mfma over butterquant int8 KV (f32 scales per row and kv head).
 hipError_t launch_prefill_full_mfma_bq(const int32_t* image, int num_qblocks, const void* q_i8,
                                        const float* qi_bias, const float* f_q, const void* k,
                                        const float* k_scale, const void* v,

@@ -29,10 +29,11 @@
 // on v_mfma_f32_16x16x32_bf16, 64 keys an iteration: two blocks fit a CU at
 // head_dim 256 and run under each other's waits.
 //
-// Measured at 16 q / 8 kv heads x 256 (us, the query-block kernel / pairs /
-// tiles): 64 tokens on 7,000 296 / 134 / 185; 500 on 7,013 484 / 140 / 192;
-// 1,000 on 7,000 513 / 278 / 250; 2,000 on 7,000 552 / 580 / 505; 32 tokens
-// decoding at 3,000 beside a 512-token chunk 374 / 191 / 157.  At 16 / 2 x 512
+// Measured at 16 q / 8 kv heads x 256 (us, prefill_pair_kernel / pairs / tiles;
+// prefill_full_mfma_kernel): 64 tokens on 7,000 270 / 134 / 185; 296.  500 on
+// 7,013 284 / 140 / 192; 484.  1,000 on 7,000 313 / 278 / 250; 513.  2,000 on
+// 7,000 361 / 580 / 505; 552.  32 tokens decoding at 3,000 beside a 512-token
+// chunk 278 / 191 / 157; 374.  At 16 / 2 x 512
 // (query-block kernel / tiles): 64 tokens 518 / 275; 500 690 / 300; 1,000 750 /
 // 580; 2,000 671 / 1,230; the mixed step 630 / 290.
 #include <type_traits>
@@ -951,7 +952,7 @@ int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, 
   };
   if (head_dim == 256) {
     const int64_t live = (seq_len + 15 * num_runs) / 16 * num_kv;
-    const double block = block_cost(num_qblocks * num_kv, 8.7, 6.5);
+    const double block = block_cost(num_qblocks * num_kv, 5.1, 6.3);
     const double pairs = 2.45 * rounds(live, 256);
     const double tiles = live <= 256 ? 3.2 : 4.3 * rounds(live, 512);
     if (block <= pairs && block <= tiles) return 0;

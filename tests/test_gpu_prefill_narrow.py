@@ -21,12 +21,16 @@ EDGES = ([0, 14, 15, 47, 62, 63, 64, 126, 127, 128, 200, 255], [2, 1, 2, 17, 1, 
 # 40 sequences of one to three tokens: more blocks than CUs at 8 kv heads.
 MANY = ([(37 * i) % 290 for i in range(40)], [1 + i % 3 for i in range(40)])
 MIXED = ([700, 31, 530, 1], [90, 1, 1, 1])
+# Enough rows for whole query blocks (64 tokens on two waves per row group).
+BLOCKS = ([0, 63, 130, 14, 200], [64, 65, 70, 50, 1])
+LONG = ([0, 63, 330], [700, 65, 300])
 
 
 @pytest.mark.parametrize("head_dim,nkv,page_len,shape", [
     (256, 8, 64, EDGES), (256, 8, 16, EDGES), (256, 8, 1024, MIXED), (256, 1, 64, MIXED),
     (256, 3, 32, EDGES), (256, 8, 64, MANY), (256, 8, 16, MANY), (512, 2, 64, EDGES),
-    (512, 2, 16, MIXED), (512, 3, 1024, EDGES), (512, 1, 64, MANY)])
+    (512, 2, 16, MIXED), (512, 3, 1024, EDGES), (512, 1, 64, MANY), (256, 32, 16, BLOCKS),
+    (256, 32, 1024, BLOCKS), (256, 8, 64, LONG)])
 def test_prefill_few_rows(head_dim, nkv, page_len, shape):
     announce(f"few-row prefill d={head_dim} kv={nkv} page={page_len} runs={len(shape[0])}")
     prefix, new = shape
