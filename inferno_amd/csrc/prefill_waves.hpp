@@ -1,5 +1,5 @@
-// Pieces of the full-attention prefill kernels whose waves share rows
-// (prefill_narrow.hip, prefill_pair.hip): lane-pair exchanges, loads into LDS
+// Pieces of the kernels whose waves share rows or stage by hand
+// (prefill_narrow.hip, prefill_pair.hip, sparse.hip): lane-pair exchanges, loads into LDS
 // with written-out waits, and the barrier that leaves loads in flight.
 #pragma once
 

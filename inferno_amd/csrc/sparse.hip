@@ -14,13 +14,14 @@
 //                       32-slot streaming bank, each reduction done as a rank
 //                       count under reduce_argmax's order (value, then slot
 //                       lane, then slot register).
-// sparse_attention_kernel  four waves per (token, kv head): S = K.Q^T and P.V
+// sparse_attention_kernel  eight waves per (token, kv head): S = K.Q^T and P.V
 //                       for the 16 q heads of the kv head on MFMA around the
-//                       reference's per-tile online softmax (each wave forms
-//                       the same scores and owns 32 output dims), then the
+//                       reference's per-tile online softmax (each wave scores
+//                       every eighth tile and owns 16 output dims), then the
 //                       one-stripe finalisation.
 #include "common.hpp"
 #include "launch.hpp"
+#include "prefill_waves.hpp"
 
 namespace ifr {
 namespace {
@@ -328,15 +329,12 @@ __global__ __launch_bounds__(256) void select_blocks_kernel(
 //
 // Scores: v_mfma_f32_16x16x32_bf16 with A = the tile's 16 keys x 32 dims and
 // B = the 16 queries' dims, so lane l holds S[pos 4*(l/16)+j][head l%16].
-// Softmax per tile follows online_softmax_tile with the biased exp; the tile
-// weight sum uses the 16-position halving tree (xor 32, xor 16, then in-lane).
-// P.V: v_mfma_f32_16x16x16_bf16 per 16-dim block with A = V^T (a transposing
-// LDS read of the tile's rows) and B = P^T, which is the softmax layout
-// itself, so the accumulator C[dim][head] rescales lane-locally.  P enters as
-// bf16 hi + lo parts (about 16 significant bits per weight); pad positions
-// carry their fexp(-87) into l but a zero weight into P.V, as in the
-// reference.  The next two tiles' keys and values load while a tile
-// computes.
+// Softmax per tile follows online_softmax_tile with the biased exp.
+// P.V: v_mfma_f32_16x16x32_bf16 over two tiles with A = V^T (transposing LDS
+// reads of their rows) and B = P^T, which is the softmax layout itself, so the
+// accumulator C[dim][head] rescales lane-locally.  P enters as bf16 hi + lo
+// parts (about 16 significant bits per weight); pad positions carry their
+// fexp(-87) into l but a zero weight into P.V, as in the reference.
 // ---------------------------------------------------------------------------
 constexpr int kSD = 128;                // head_dim
 constexpr int kSG = 16;                 // q heads per kv head
@@ -377,30 +375,38 @@ __device__ __forceinline__ TileCursor next_tile(TileCursor c, const int32_t* bro
   return c;
 }
 
-struct TileRegs {
-  uint4 k0, k1, k2, k3;  // keys: row r16, dims 32c + 8g .. +8
-  uint4 v0;              // values: row lane/4, 16 bytes of the wave's 32 dims
-};
-// The four waves of a workgroup share one (token, kv head): each forms the
-// same scores and softmax (identical arithmetic) and owns 32 of the 128
-// output dims in P.V, so a decode step has four times as many waves on its
-// block lists.  V rows of the wave's dims are staged at a 96-byte pitch
-// (4 rows x 32 bytes of a transposing read fall on distinct banks).
-constexpr int kSDW = kSD / 4;                 // output dims per wave
-constexpr int kSVPitchW = kSDW * 2 + 32;      // bytes per V row in LDS
-constexpr int kSVBytesW = kTile * kSVPitchW;
+// Eight waves share one (token, kv head), eight tiles an iteration:
+//
+//   scores   wave w takes tile w of the iteration, S = K.Q^T
+//   softmax  the tile maxima go through LDS; every wave then knows the running
+//            maximum before and after each tile, so each takes its own tile's
+//            weights at once, scaled by the later tiles' corrections
+//   P.V      wave w owns output dims 16 w .. +15 and reads all tiles' values and
+//            weights (bf16 hi + lo parts) from LDS
+//
+// A tile's keys and values stay in registers from their load, two iterations
+// ahead, to their use: 64 to 128 KB in flight for each CU, and bound by HBM there.
+// Measured against four waves that each walked every tile for a quarter of the
+// dims (32 KB in flight, every tile's softmax in line): 64 tokens x 4 kv heads x
+// 16 blocks of 128 89 -> 54 us (268 MB, 5.0 TB/s), one token 84 -> 42, 512 tokens
+// 495 -> 226 (345 at one workgroup a CU, so the 128 registers of two).
+constexpr int kSWaves = 8;
+constexpr uint32_t kNoTile = 0x7FC0ABCDu;  // a tile maximum: no position (a NaN no score has)
 
-__global__ __launch_bounds__(256) void sparse_attention_kernel(
+__global__ __launch_bounds__(64 * kSWaves) __attribute__((amdgpu_waves_per_eu(4, 4)))
+void sparse_attention_kernel(
     const int32_t* __restrict__ image, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ k_base, const uint16_t* __restrict__ v_base,
     const int32_t* __restrict__ block_idx, uint16_t* __restrict__ out, int64_t kv_stride,
-    int num_q, int num_kv, int block_size, int topk, int shift, int row_mask, int num_rows) {
-  __shared__ __align__(16) uint8_t vlds[4][2][kSVBytesW];
+    int num_q, int num_kv, int block_size, int topk, int shift, int row_mask) {
+  __shared__ __align__(16) uint8_t vlds[kSWaves][kSVBytes];
+  __shared__ __align__(16) uint4 q_lds[4][64];
+  __shared__ __align__(16) uint2 p_lds[2][kSWaves / 2][64][2];  // hi and lo, by tile pair
+  __shared__ __align__(16) uint32_t tmax_lds[kSG][kSWaves];
+  __shared__ __align__(16) float tsum_lds[kSG][kSWaves];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x;
-  if (row >= num_rows) return;
-  const int dq = wave;  // the wave's quarter of the output dims
   const int t = row / num_kv;
   const int h = row - t * num_kv;
   const TokenPos tp = token_position(image, t);
@@ -408,174 +414,182 @@ __global__ __launch_bounds__(256) void sparse_attention_kernel(
   const int r16 = lane & 15;
   const int g = lane >> 4;
 
-  // B operand of the scores: Q[head r16][32c + 8g .. +8] for c = 0..3.
-  bf16x8_t qf[4];
-  {
-    const uint16_t* qrow =
-        q + (static_cast<int64_t>(t) * num_q + h * kSG + r16) * kSD + 8 * g;
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      qf[c] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qrow + 32 * c));
-  }
-  const uint16_t* kh = k_base + static_cast<int64_t>(h) * kSD;
-  const uint16_t* vh = v_base + static_cast<int64_t>(h) * kSD;
+  // The list ends at its first -1.
   const int32_t* brow = block_idx + static_cast<int64_t>(row) * topk;
-  // V staging: lane takes 16 bytes (chunk lane%4) of row lane/4 of the
-  // wave's 32 dims.
-  const int vrow_l = lane >> 2;
-  const int vcol = 16 * (lane & 3);
-  // Transposing read: lane r16 of group g addresses row 4g + r16/4, dims
-  // 4*(r16%4) .. +3 of a 16-dim block, and receives V[4g + k][16b + r16].
-  const int tr_off = (4 * g + (r16 >> 2)) * kSVPitchW + 8 * (r16 & 3);
+  int n_slots = topk;
+  for (int s0 = 0; s0 < topk; s0 += 64) {
+    const uint64_t ends = __builtin_amdgcn_ballot_w64(s0 + lane < topk && brow[min(s0 + lane, topk - 1)] < 0);
+    if (ends) {
+      n_slots = s0 + __builtin_ctzll(ends);
+      break;
+    }
+  }
 
-  // A tile never straddles a page (page_len >= 16, tiles 16-aligned), so its
-  // page row is one uniform (scalar) load, not a vector load the K/V loads
-  // would have to wait behind.
-  auto page_row = [&](const TileCursor& c) -> int64_t {
-    return sload(tp.rows + static_cast<int>(c.pos >> shift));
+  // B operand of the scores, from LDS (in registers, it would not leave room for
+  // the loads in flight at 128 a wave): Q[head r16][32c + 8g .. +8] for c = 0..3.
+  if (wave < 4)
+    q_lds[wave][lane] = *reinterpret_cast<const uint4*>(
+        q + (static_cast<int64_t>(t) * num_q + h * kSG + r16) * kSD + 32 * wave + 8 * g);
+  const uint16_t* kh = k_base + static_cast<int64_t>(h) * kSD + 8 * g;
+  const uint16_t* vh = v_base + static_cast<int64_t>(h) * kSD + 8 * r16;
+
+  // The wave's tiles: number wave, wave + 8, ... of the list's, every block
+  // counted with all its tiles (at most those of the context).  Those past the
+  // causal end, or past the list, have no position and change nothing.
+  const int tpb = static_cast<int>(min<int64_t>(block_size / kTile, (cap + kTile - 1) / kTile));
+  const int step_s = kSWaves / tpb, step_sub = kSWaves % tpb;
+  int slot = wave / tpb, sub = wave % tpb;
+  struct Tile {
+    int len;
+    int64_t row;  // cache row of its first position (no position: the sequence's first)
   };
-  auto load_tile = [&](const TileCursor& c, int64_t prow) {
-    TileRegs d;
-    const int tl = static_cast<int>(min<int64_t>(kTile, c.phi - c.pos));
-    const int off0 = static_cast<int>(c.pos) & row_mask;
-    const int64_t kslot = prow + off0 + (r16 < tl ? r16 : 0);
-    const uint16_t* kp = kh + kslot * kv_stride + 8 * g;
-    d.k0 = *reinterpret_cast<const uint4*>(kp);
-    d.k1 = *reinterpret_cast<const uint4*>(kp + 32);
-    d.k2 = *reinterpret_cast<const uint4*>(kp + 64);
-    d.k3 = *reinterpret_cast<const uint4*>(kp + 96);
-    const int64_t vslot = prow + off0 + (vrow_l < tl ? vrow_l : 0);
-    d.v0 = *reinterpret_cast<const uint4*>(
-        reinterpret_cast<const uint8_t*>(vh + vslot * kv_stride + kSDW * dq) + vcol);
+  // A tile never straddles a page (page_len >= 16, tiles 16-aligned), so its
+  // page row is one uniform (scalar) load, a step ahead of the loads that use it.
+  auto next_of_wave = [&]() {
+    int64_t pos = cap;
+    int64_t end = cap;
+    if (slot < n_slots) {
+      const int64_t first = static_cast<int64_t>(sload(brow + slot)) * block_size;
+      pos = first + kTile * sub;
+      end = min(first + block_size, cap);
+    }
+    Tile d;
+    d.len = static_cast<int>(max<int64_t>(0, min<int64_t>(kTile, end - pos)));
+    const int at = d.len > 0 ? static_cast<int>(pos) : 0;
+    d.row = static_cast<int64_t>(sload(tp.rows + (at >> shift))) + (at & row_mask);
+    slot += step_s;
+    sub += step_sub;
+    if (sub >= tpb) {
+      sub -= tpb;
+      ++slot;
+    }
     return d;
   };
-
-  float m = kNegBig;  // state of head r16 (the same in its four lanes)
-  float lsum = 0.0f;
-  f32x4_t acc[kSDW / 16];  // acc[b][j] = O[dim 32dq + 16b + 4g + j][head r16]
-#pragma unroll
-  for (int b = 0; b < kSDW / 16; ++b) acc[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-  // A tile's scores and softmax, then P.V; between the two the caller
-  // reuses the tile's registers for the loads of a later tile.
-  auto scores = [&](const TileRegs& rg, const TileCursor& c, int buf) {
-    uint8_t* vb = vlds[wave][buf];
-    wave_sync();
-    *reinterpret_cast<uint4*>(vb + vrow_l * kSVPitchW + vcol) = rg.v0;
-    f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
-    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rg.k0), qf[0], sc, 0, 0, 0);
-    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rg.k1), qf[1], sc, 0, 0, 0);
-    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rg.k2), qf[2], sc, 0, 0, 0);
-    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rg.k3), qf[3], sc, 0, 0, 0);
-    return sc;
+  struct Regs {
+    uint4 k[4];  // keys: row r16, dims 32c + 8g .. +8
+    uint4 v[4];  // values: row 4i + g, dims 8 r16 .. +8
+    int len;
   };
-  auto softmax_pv = [&](const f32x4_t& sc, const TileCursor& c, int buf) {
-    const int tl = static_cast<int>(min<int64_t>(kTile, c.phi - c.pos));
-    uint8_t* vb = vlds[wave][buf];
+  // Rows past a tile's last position repeat its first (in bounds).
+  auto load_tile = [&](Regs& d, const Tile& c) {
+    d.len = c.len;
+    const uint16_t* kp = kh + (c.row + (r16 < c.len ? r16 : 0)) * kv_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d.k[i] = *reinterpret_cast<const uint4*>(kp + 32 * i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int vr = 4 * i + g;
+      d.v[i] = *reinterpret_cast<const uint4*>(vh + (c.row + (vr < c.len ? vr : 0)) * kv_stride);
+    }
+  };
+
+  float m = kNegBig;  // state of head r16 (the same in its four lanes and all waves)
+  float lsum = 0.0f;
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};  // acc[j] = O[dim 16 wave + 4g + j][head r16]
+
+  const int n_it = static_cast<int>((static_cast<int64_t>(n_slots) * tpb + kSWaves - 1) / kSWaves);
+  Regs sets[2];
+  load_tile(sets[0], next_of_wave());
+  __builtin_amdgcn_sched_barrier(0);
+  load_tile(sets[1], next_of_wave());
+  __builtin_amdgcn_sched_barrier(0);
+  Tile pend = next_of_wave();
+  prefill::lds_barrier();
+
+  auto iteration = [&](Regs& rg) {
+    const int len = rg.len;
+    f32x4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(bf16x8_t, rg.k[c]),
+          __builtin_bit_cast(bf16x8_t, q_lds[c][lane]), sc, 0, 0, 0);
     // Scores of pad positions are -1e30 (their fexp(-87) enters l only).
     float sj[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sj[j] = (4 * g + j < tl) ? sc[j] : kNegBig;
-    float tmax = max_ref(max_ref(sj[0], sj[1]), max_ref(sj[2], sj[3]));
-    tmax = pair_max32(pair_max16(tmax));  // lane swaps, not LDS permutes
-    const float m_new = tmax > m ? tmax : m;
-    const float corr = fexp(max_ref(-87.0f, m - m_new));
+    for (int j = 0; j < 4; ++j) sj[j] = (4 * g + j < len) ? sc[j] : kNegBig;
+    const float tmax = pair_max32(pair_max16(max_ref(max_ref(sj[0], sj[1]), max_ref(sj[2], sj[3]))));
+    if (g == 0) tmax_lds[r16][wave] = len > 0 ? __float_as_uint(tmax) : kNoTile;
+    prefill::lds_barrier();
+
+    // Values into LDS (zeros for a tile without a position: its weights are 0,
+    // the row that was loaded for it is not its own), and the set's next loads.
+    uint8_t* vw = vlds[wave] + g * kSVPitch + 16 * r16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<uint4*>(vw + 4 * i * kSVPitch) = len > 0 ? rg.v[i] : make_uint4(0, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_tile(rg, pend);
+    __builtin_amdgcn_sched_barrier(0);
+    pend = next_of_wave();
+
+    // Corrections of the eight tiles in order, the product of all, and of those
+    // after the wave's own.
+    float total = 1.0f, after = 1.0f, m_own = m;
+#pragma unroll
+    for (int i = 0; i < kSWaves; ++i) {
+      const uint32_t bits = tmax_lds[r16][i];
+      const float ti = __uint_as_float(bits);
+      const float m_new = ti > m ? ti : m;  // kNoTile compares false
+      const float c = bits == kNoTile ? 1.0f : fexp(max_ref(-87.0f, m - m_new));
+      total = total * c;
+      after = i > wave ? after * c : after;
+      m_own = i == wave ? m_new : m_own;
+      m = m_new;
+    }
     float w[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = fexp(max_ref(-87.0f, sj[j] - m_new));
-    // 16-position halving tree: t with t+8 (xor 32), t+4 (xor 16), then j+2, j+1.
-    float ws[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) ws[j] = pair_sum16(pair_sum32(w[j]));
-    const float wsum = (ws[0] + ws[2]) + (ws[1] + ws[3]);
-    lsum = lsum * corr + wsum;
-    m = m_new;
+    for (int j = 0; j < 4; ++j)
+      w[j] = len > 0 ? fexp(max_ref(-87.0f, sj[j] - m_own)) * after : 0.0f;
+    const float wsum = pair_sum16(pair_sum32((w[0] + w[2]) + (w[1] + w[3])));
+    if (g == 0) tsum_lds[r16][wave] = wsum;
     // P^T as bf16 hi + lo, zero at pads.
-    s16x4_t phi, plo;
+    uint32_t hi[2], lo[2];
 #pragma unroll
     for (int j = 0; j < 4; j += 2) {
-      const float p0 = (4 * g + j < tl) ? w[j] : 0.0f;
-      const float p1 = (4 * g + j + 1 < tl) ? w[j + 1] : 0.0f;
+      const float p0 = (4 * g + j < len) ? w[j] : 0.0f;
+      const float p1 = (4 * g + j + 1 < len) ? w[j + 1] : 0.0f;
       const bf16x2_t hb = __builtin_convertvector(f32x2_t{p0, p1}, bf16x2_t);
       const float r0 = p0 - static_cast<float>(hb[0]);
       const float r1 = p1 - static_cast<float>(hb[1]);
       const bf16x2_t lb = __builtin_convertvector(f32x2_t{r0, r1}, bf16x2_t);
-      const s16x4_t hs = __builtin_bit_cast(s16x4_t, __builtin_shufflevector(hb, hb, 0, 1, 0, 1));
-      const s16x4_t ls = __builtin_bit_cast(s16x4_t, __builtin_shufflevector(lb, lb, 0, 1, 0, 1));
-      phi[j] = hs[0];
-      phi[j + 1] = hs[1];
-      plo[j] = ls[0];
-      plo[j + 1] = ls[1];
+      hi[j / 2] = __builtin_bit_cast(uint32_t, hb);
+      lo[j / 2] = __builtin_bit_cast(uint32_t, lb);
     }
-    wave_sync();
-#pragma unroll
-    for (int b = 0; b < kSDW / 16; ++b) {
-      acc[b] = acc[b] * corr;  // scale_unrolled for head r16
-      const s16x4_t va =
-          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vb + tr_off + 32 * b));
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, phi, acc[b], 0, 0, 0);
-      acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va, plo, acc[b], 0, 0, 0);
-    }
-  };
+    p_lds[0][wave >> 1][lane][wave & 1] = make_uint2(hi[0], hi[1]);
+    p_lds[1][wave >> 1][lane][wave & 1] = make_uint2(lo[0], lo[1]);
+    prefill::lds_barrier();
 
-  // kAhead tiles in flight in rotating register sets (no copies between
-  // them): set s holds tile i + s; once tile i's scores have read its keys
-  // and its values are in LDS, the set takes the loads of tile i + kAhead.
-  // The loads are unconditional -- past the block list they all read the
-  // sequence's first row (in bounds, unused) -- so every step leaves the same
-  // loads in flight and each wait covers only older loads.  The next
-  // cursor's page row is read (scalar) one step before its loads use it.
-  // An even depth keeps each step's LDS buffer a compile-time choice
-  // (measured: depths 2 and 4 93 us, 3 and 5 100 us, 6 and 8 98.5 us).
-  constexpr int kAhead = 4;
-  auto advance = [&](const TileCursor& c) {
-    return c.valid ? next_tile(c, brow, topk, block_size, cap) : c;
-  };
-  auto dummy_or = [&](const TileCursor& c) {
-    TileCursor d = c;  // selects, not a branch: one code path for the loads
-    d.pos = c.valid ? c.pos : 0;
-    d.phi = c.valid ? c.phi : kTile;
-    return d;
-  };
-  TileCursor cs[kAhead];
-  TileRegs rs[kAhead];
-  cs[0] = next_tile(TileCursor{-1, 0, 0, false}, brow, topk, block_size, cap);
+    acc = acc * total;
+    lsum = lsum * total;
+    const float4 s0 = *reinterpret_cast<const float4*>(&tsum_lds[r16][0]);
+    const float4 s1 = *reinterpret_cast<const float4*>(&tsum_lds[r16][4]);
+    lsum = lsum + (((s0.x + s0.y) + (s0.z + s0.w)) + ((s1.x + s1.y) + (s1.z + s1.w)));
+    // Two tiles an MFMA: values 0..3 of a lane are positions 4g .. +3 of the
+    // first, 4..7 of the second.  Transposing read: lane r16 of group g addresses
+    // row 4g + r16/4, dims 4*(r16%4) .. +3 of the wave's 16.
+    const uint8_t* vr = &vlds[0][0] + (4 * g + (r16 >> 2)) * kSVPitch + 32 * wave + 8 * (r16 & 3);
 #pragma unroll
-  for (int i = 1; i < kAhead; ++i) cs[i] = advance(cs[i - 1]);
-  // Issued in set order, as the loop issues them (the waits count on it).
+    for (int pr = 0; pr < kSWaves / 2; ++pr) {
+      const s16x4_t v0 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vr + 2 * pr * kSVBytes));
+      const s16x4_t v1 =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vr + (2 * pr + 1) * kSVBytes));
+      const bf16x8_t va = __builtin_bit_cast(
+          bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-  for (int i = 0; i < kAhead; ++i) {
-    const TileCursor d = dummy_or(cs[i]);
-    rs[i] = load_tile(d, page_row(d));
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  TileCursor pend = dummy_or(advance(cs[kAhead - 1]));  // the next tile to issue
-  bool pend_valid = advance(cs[kAhead - 1]).valid;
-  TileCursor last = advance(cs[kAhead - 1]);
-  int64_t pend_row = page_row(pend);
-  int buf = 0;
-  for (;;) {
-#pragma unroll
-    for (int s = 0; s < kAhead; ++s) {
-      // Leaving the loop is the only branch: every path that goes on has
-      // issued the same loads.
-      if (!cs[s].valid) goto tiles_done;  // uniform
-      const TileCursor c = cs[s];
-      const f32x4_t sc = scores(rs[s], c, buf);
-      __builtin_amdgcn_sched_barrier(0);
-      rs[s] = load_tile(pend, pend_row);
-      __builtin_amdgcn_sched_barrier(0);
-      cs[s] = pend;
-      cs[s].valid = pend_valid;
-      last = advance(last);
-      pend_valid = last.valid;
-      pend = dummy_or(last);
-      pend_row = page_row(pend);
-      softmax_pv(sc, c, buf);
-      buf ^= 1;
+      for (int part = 0; part < 2; ++part) {
+        const bf16x8_t pb = __builtin_bit_cast(
+            bf16x8_t, *reinterpret_cast<const uint4*>(&p_lds[part][pr][lane][0]));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb, acc, 0, 0, 0);
+      }
     }
+  };
+  for (int it = 0; it < n_it; it += 2) {
+    iteration(sets[0]);
+    if (it + 1 >= n_it) break;  // uniform over the block
+    iteration(sets[1]);
   }
-tiles_done:
 
   // write_finalized_head over one stripe: cv = fexp(0) scales both acc and
   // l (l > 0), out = (acc * cv) * (1 / (0 + l * cv)).
@@ -584,17 +598,13 @@ tiles_done:
   cv = lsum > 0.0f ? cv : 0.0f;
   const float gl = 0.0f + lsum * cv;
   const float inv = gl > 0.0f ? 1.0f / gl : 0.0f;
-  uint16_t* orow =
-      out + (static_cast<int64_t>(t) * num_q + h * kSG + r16) * kSD + kSDW * dq + 4 * g;
-#pragma unroll
-  for (int b = 0; b < kSDW / 16; ++b) {
-    uint32_t lo = 0, hi = 0;
-    if (gl > 0.0f) {
-      lo = f32_to_bf16_bits((acc[b][0] * cv) * inv) | (f32_to_bf16_bits((acc[b][1] * cv) * inv) << 16);
-      hi = f32_to_bf16_bits((acc[b][2] * cv) * inv) | (f32_to_bf16_bits((acc[b][3] * cv) * inv) << 16);
-    }
-    *reinterpret_cast<uint2*>(orow + 16 * b) = make_uint2(lo, hi);
+  uint16_t* orow = out + (static_cast<int64_t>(t) * num_q + h * kSG + r16) * kSD + 16 * wave + 4 * g;
+  uint32_t o0 = 0, o1 = 0;
+  if (gl > 0.0f) {
+    o0 = f32_to_bf16_bits((acc[0] * cv) * inv) | (f32_to_bf16_bits((acc[1] * cv) * inv) << 16);
+    o1 = f32_to_bf16_bits((acc[2] * cv) * inv) | (f32_to_bf16_bits((acc[3] * cv) * inv) << 16);
   }
+  *reinterpret_cast<uint2*>(orow) = make_uint2(o0, o1);
 }
 
 // ---------------------------------------------------------------------------
@@ -881,6 +891,10 @@ struct BqSplitRegs {
   float ks[4], vs[4];  // scales of positions 4g + j
 };
 constexpr int kSAhead = 4;
+
+constexpr int kSDW = kSD / 4;                 // output dims per wave
+constexpr int kSVPitchW = kSDW * 2 + 32;      // bytes per V row in LDS
+constexpr int kSVBytesW = kTile * kSVPitchW;
 
 __global__ __launch_bounds__(256) void bq_sparse_split_kernel(
     const int32_t* __restrict__ image, const int8_t* __restrict__ q_i8,
@@ -1211,11 +1225,11 @@ hipError_t launch_block_sparse_attention(const int32_t* image, int seq_len, cons
                                          hipStream_t stream) {
   if (seq_len <= 0) return hipSuccess;
   const int rows = seq_len * num_kv;
-  hipLaunchKernelGGL(sparse_attention_kernel, dim3(rows), dim3(256), 0, stream,
+  hipLaunchKernelGGL(sparse_attention_kernel, dim3(rows), dim3(64 * kSWaves), 0, stream,
                      image, static_cast<const uint16_t*>(q),
                      static_cast<const uint16_t*>(k_base), static_cast<const uint16_t*>(v_base),
                      block_idx, static_cast<uint16_t*>(output), kv_stride, num_q, num_kv,
-                     block_size, topk, shift, row_mask, rows);
+                     block_size, topk, shift, row_mask);
   return hipGetLastError();
 }
 

@@ -295,3 +295,48 @@ def test_bq_sparse_batched_decode_on_indexer_selection(page_len):
     inputs = _bq_inputs(rng, len(ctx), case.cache_rows)
     r = _check_bq_sparse(plan, case.runs, case.base_rows, inputs, bi, page_len, cap=8)
     print(f"  bq sparse batched decode vs oracle: {r}", flush=True)
+
+
+EDGE_CTX = [0, 14, 15, 16, 30, 31, 32, 62, 63, 64, 95, 127, 128, 129, 159, 255, 256, 700, 1023, 2100]
+
+
+@pytest.mark.parametrize("block,page_len,topk", [(64, 64, 16), (128, 64, 3), (192, 1024, 5),
+                                                 (96, 64, 16), (16, 16, 32), (48, 16, 1)])
+def test_block_and_round_edges(block, page_len, topk):
+    """Contexts around the edges of tiles (16), half rounds (32), rounds (64) and
+    blocks, index blocks that are and are not whole rounds, blocks of fewer tiles
+    than waves.  Block ids are exact; the attention on them within 1e-2.  Every row
+    past a sequence's last position holds NaN."""
+    announce(f"sparse edges block={block} page={page_len} topk={topk}")
+    rng = np.random.default_rng(block + topk)
+    n = len(EDGE_CTX)
+    case = make_decode_case(31, EDGE_CTX, page_len=page_len)
+    used = np.zeros(case.cache_rows, dtype=bool)
+    for pages, c in zip(case.pages, EDGE_CTX):
+        used[np.concatenate([np.arange(page_len) + g * page_len for g in pages])[:c + 1]] = True
+
+    def poisoned(x):
+        x = x.reshape(case.cache_rows, -1).copy()
+        x[~used] = 0x7FC0
+        return to_dev(x)
+
+    index_q = _bf(rng.standard_normal(n * IH * HD))
+    index_k = _bf(rng.standard_normal(case.cache_rows * HD))
+    q, k, v = _sparse_inputs(rng, n, case.cache_rows)
+    plan = _plan(case.runs, case.base_rows, n, case.cache_rows, page_len)
+    bi = empty_dev(n * IH * topk, np.int32)
+    out = empty_dev(n * NUM_Q * HD, np.uint16)
+    A.dispatch_lightning_indexer(plan, to_dev(index_q), poisoned(index_k), bi,
+                                 A.index_scores_buffer(plan, IH, block), block_size=block,
+                                 topk_blocks=topk)
+    A.dispatch_block_sparse_attention(plan, to_dev(q), poisoned(k), poisoned(v), bi, out,
+                                      block_size=block, topk_blocks=topk)
+    got = from_dev(bi, np.int32).reshape(n, IH, topk)
+    want, _ = oracle.lightning_indexer(case.runs, case.base_rows, index_q, index_k, num_heads=IH,
+                                       head_dim=HD, block_size=block, topk=topk, local_blocks=1,
+                                       init_blocks=0, scale=SCALE, page_len=page_len, seq_len=n)
+    assert np.array_equal(got, want), np.argwhere(got != want)[:5]
+    ref = oracle.block_sparse_attention(case.runs, case.base_rows, q, k, v, want, num_q=NUM_Q,
+                                        num_kv=NUM_KV, head_dim=HD, kv_stride=KV_STRIDE,
+                                        block_size=block, topk=topk, page_len=page_len, seq_len=n)
+    assert_bar(compare_bf16(from_dev(out, np.uint16), ref), f"sparse edges block={block}")
