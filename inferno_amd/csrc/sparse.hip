@@ -53,13 +53,84 @@ __device__ __forceinline__ TokenPos token_position(const int32_t* image, int t) 
 // (32p + 2j + 1, 32p + 2j) as odd*odd + even*even, lane j sums its
 // accumulators p = 0.. in order, then the 16-lane halving tree.
 // ---------------------------------------------------------------------------
+// Strips kP0 .. +kNP - 1 of a position per lane (kv: that part of its key) against
+// all heads' queries.  The key's pairs are unpacked once; the queries are
+// wave-uniform, bf16 pairs read as scalar dwords and unpacked on the SALU, so each
+// FMA takes its query value from an SGPR (no LDS staging or reads).
+template <int D, int H, int kP0, int kNP>
+__device__ __forceinline__ void score_strips(const uint4 (&kv)[4 * kNP],
+                                             const int32_t* qg, float (&s)[H][16]) {
+  // A strip's 16 dwords of a head, read one (strip, head) ahead.  The reads and the
+  // sums are held in place: left to the compiler they are hoisted, and 256 dwords
+  // go through VGPR lanes (a third of the round's instructions).
+  uint32_t qw[2][16];
+  auto read_q = [&](int i) {
+    asm volatile("" : "+s"(qg));
+    const int32_t* src = qg + ((i % H) * D + 32 * (kP0 + i / H)) / 2;  // pairs j = 0..15
+#pragma unroll
+    for (int j = 0; j < 16; ++j) qw[i & 1][j] = static_cast<uint32_t>(sload(src + j));
+  };
+  read_q(0);
+#pragma unroll
+  for (int p = 0; p < kNP; ++p) {
+    float klo[16], khi[16];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint4 v = kv[4 * p + c];
+      const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        klo[4 * c + e] = bf16_lo(w4[e]);
+        khi[4 * c + e] = bf16_hi(w4[e]);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int i = p * H + h;
+      uint32_t (&w)[16] = qw[i & 1];
+      // Scalar loads return in any order: this head's are waited for before the
+      // next ones are issued.
+      asm volatile("" ::"s"(w[0]), "s"(w[1]), "s"(w[2]), "s"(w[3]), "s"(w[4]), "s"(w[5]), "s"(w[6]),
+                   "s"(w[7]), "s"(w[8]), "s"(w[9]), "s"(w[10]), "s"(w[11]), "s"(w[12]),
+                   "s"(w[13]), "s"(w[14]), "s"(w[15]));
+      if (i + 1 < kNP * H) read_q(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const float qe = __uint_as_float(w[j] << 16), qo = __uint_as_float(w[j] & 0xFFFF0000u);
+        // bf16 products are exact in f32, so the fma rounds (odd + even) once.
+        const float a = fmaf(klo[j], qe, khi[j] * qo);
+        s[h][j] = kP0 + p == 0 ? a : s[h][j] + a;
+      }
+      float (&r)[16] = s[h];
+      asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]),
+                   "+v"(r[6]), "+v"(r[7]), "+v"(r[8]), "+v"(r[9]), "+v"(r[10]), "+v"(r[11]),
+                   "+v"(r[12]), "+v"(r[13]), "+v"(r[14]), "+v"(r[15]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+// The halving trees, and the lane's running maxima.
+template <int H>
+__device__ __forceinline__ void score_maxima(float (&s)[H][16], float scale, bool valid,
+                                             float (&best)[H]) {
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+#pragma unroll
+    for (int w = 8; w >= 1; w >>= 1) {
+#pragma unroll
+      for (int jj = 0; jj < w; ++jj) s[h][jj] = s[h][jj] + s[h][jj + w];
+    }
+    const float sh = s[h][0] * scale;
+    best[h] = valid && sh > best[h] ? sh : best[h];
+  }
+}
+
 template <int D, int H, bool kPageRows>
 __global__ __launch_bounds__(256) void index_scores_kernel(
     const int32_t* __restrict__ image, const uint16_t* __restrict__ index_q,
     const uint16_t* __restrict__ index_k, float* __restrict__ scores, int block_stride,
     int block_size, float scale, int shift, int row_mask) {
-  constexpr int kP = D / 32;  // port-unroll accumulators, one strip
-  static_assert(H * D == 64 * 8, "one 16-byte query load per lane");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.y;
@@ -92,58 +163,15 @@ __global__ __launch_bounds__(256) void index_scores_kernel(
   };
   uint4 kv[D / 8];
   load_round(lo, kv);
-  // The token's queries are wave-uniform: bf16 pairs read as scalar dwords
-  // and unpacked on the SALU, so each FMA takes its query value from an
-  // SGPR (no LDS staging or reads).
   const int32_t* qg = reinterpret_cast<const int32_t*>(index_q + static_cast<int64_t>(t) * H * D);
   float best[H];
 #pragma unroll
   for (int h = 0; h < H; ++h) best[h] = kNegBig;
-  // A lane takes whole positions and all heads: the key's pairs are unpacked
-  // once, the queries are read from LDS (every lane the same address).
   for (int p0 = lo; p0 < hi; p0 += 64) {
     const bool valid = p0 + lane < hi;
-    // The query reads stay inside the loop (hoisted, 256 dwords would not
-    // fit in SGPRs).
-    int qoff = 0;
-    asm volatile("" : "+s"(qoff));
     float s[H][16];
-#pragma unroll
-    for (int p = 0; p < kP; ++p) {
-      float klo[16], khi[16];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint4 v = kv[4 * p + c];
-        const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          klo[4 * c + e] = bf16_lo(w4[e]);
-          khi[4 * c + e] = bf16_hi(w4[e]);
-        }
-      }
-#pragma unroll
-      for (int h = 0; h < H; ++h) {
-        const int32_t* qh = qg + qoff + (h * D + 32 * p) / 2;  // 16 dwords: pairs j = 0..15
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const uint32_t qw = static_cast<uint32_t>(sload(qh + j));
-          const float qe = __uint_as_float(qw << 16), qo = __uint_as_float(qw & 0xFFFF0000u);
-          // bf16 products are exact in f32, so the fma rounds (odd + even) once.
-          const float a = fmaf(klo[j], qe, khi[j] * qo);
-          s[h][j] = p == 0 ? a : s[h][j] + a;
-        }
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-#pragma unroll
-      for (int w = 8; w >= 1; w >>= 1) {
-#pragma unroll
-        for (int jj = 0; jj < w; ++jj) s[h][jj] = s[h][jj] + s[h][jj + w];
-      }
-      const float sh = s[h][0] * scale;
-      best[h] = valid && sh > best[h] ? sh : best[h];
-    }
+    score_strips<D, H, 0, D / 32>(kv, qg, s);
+    score_maxima<H>(s, scale, valid, best);
     // The next round's loads are issued after this round's math (with its
     // registers, 3 waves fit per SIMD; a prefetch into a second set, at 2
     // waves per SIMD, measured slower).
@@ -154,6 +182,89 @@ __global__ __launch_bounds__(256) void index_scores_kernel(
     float v = best[h];
 #pragma unroll
     for (int msk = 1; msk < 64; msk <<= 1) v = fmaxf(v, shfl_xor_f32(v, msk));
+    if (lane == 0) scores[(static_cast<int64_t>(t) * H + h) * block_stride + b] = v;
+  }
+}
+
+// The same scores where a round of 64 positions never leaves a page (pages and
+// index blocks of whole rounds), one wave a workgroup and index block.  Half rows
+// of a round's 64 (128 bytes each) enter LDS by 1 KB loads and a lane reads its
+// own back (chunk c of row r at c ^ (r / 2 % 8)); a half is in registers before
+// its math, so LDS takes the next one meanwhile.  In index_scores_kernel a 16-byte
+// load touches 64 rows and is waited for by the wave that issued it.
+//
+// Bound by VALU issue (256 multiplies, 256 FMAs and 192 adds a position in the
+// reference's order; v_dot2_f32_bf16 rounds otherwise) where keys come from cache,
+// by HBM where they do not.  Measured against index_scores_kernel, with the
+// selection: 64 tokens on 1,024 to 131,071 keys 242 -> 216 us, 16 on up to 60,000
+// 51 -> 46, one on 30,000 29.4 -> 26.4, 512 tokens of one sequence on 20,000
+// 380 -> 263.  Four waves a SIMD (12 fewer registers than needed) 287 us, several
+// blocks a wave 224 to 253.
+template <int D, int H>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
+void index_scores_rounds_kernel(
+    const int32_t* __restrict__ image, const uint16_t* __restrict__ index_q,
+    const uint16_t* __restrict__ index_k, float* __restrict__ scores, int block_stride,
+    int block_size, float scale, int shift, int row_mask) {
+  static_assert(D == 128, "two halves of 8 chunks");
+  __shared__ __align__(16) uint8_t rows[64 * D];
+  const int lane = threadIdx.x;
+  const int t = blockIdx.y;
+  const TokenPos tp = token_position(image, t);
+  const int b = blockIdx.x;
+  if (b >= min(tp.abs_pos / block_size + 1, block_stride)) return;
+  const int lo = b * block_size;
+  const int hi = min(lo + block_size, tp.abs_pos + 1);
+
+  // Load i of a half: rows 8 i .. +7 of 32 (the instruction's own offset, 1024 i,
+  // counts on both sides).
+  uint32_t off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    off[i] = static_cast<uint32_t>((lane >> 3) * D * 2 + 1024 * i +
+                                   16 * ((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)));
+  // Up to 31 rows past hi come along (the same page's); their scores are dropped.
+  auto load_half = [&](int64_t slot, int half, bool upper) {
+    const char* src = reinterpret_cast<const char*>(index_k) + slot * (D * 2) + half * D;
+    prefill::load_lds4(src, off[0], off[1], off[2], off[3], rows);
+    if (upper)
+      prefill::load_lds4(src + 32 * D * 2, off[0], off[1], off[2], off[3], rows + 32 * D);
+  };
+  auto slot_of = [&](int pos) {
+    return static_cast<int64_t>(sload(tp.rows + (pos >> shift))) + (pos & row_mask);
+  };
+  const uint8_t* mine = rows + lane * D;
+  auto read_half = [&](uint4 (&kv)[D / 16]) {
+    prefill::wait_loads<0>();
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c)
+      kv[c] = *reinterpret_cast<const uint4*>(mine + 16 * (c ^ ((lane >> 1) & 7)));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the half is in registers
+  };
+
+  const int32_t* qg = reinterpret_cast<const int32_t*>(index_q + static_cast<int64_t>(t) * H * D);
+  float best[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) best[h] = kNegBig;
+  int64_t slot = slot_of(lo);
+  load_half(slot, 0, lo + 32 < hi);
+  for (int p0 = lo; p0 < hi; p0 += 64) {
+    uint4 kv[D / 16];
+    float s[H][16];
+    read_half(kv);
+    load_half(slot, 1, p0 + 32 < hi);
+    score_strips<D, H, 0, D / 64>(kv, qg, s);
+    read_half(kv);
+    if (p0 + 64 < hi) {
+      slot = slot_of(p0 + 64);
+      load_half(slot, 0, p0 + 96 < hi);
+    }
+    score_strips<D, H, D / 64, D / 64>(kv, qg, s);
+    score_maxima<H>(s, scale, p0 + lane < hi, best);
+  }
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const float v = wave_max_ref(best[h]);
     if (lane == 0) scores[(static_cast<int64_t>(t) * H + h) * block_stride + b] = v;
   }
 }
@@ -1156,7 +1267,11 @@ hipError_t launch_lightning_indexer(const int32_t* image, int seq_len, const voi
   dim3 grid((block_stride + 3) / 4, seq_len);
   const auto* iq = static_cast<const uint16_t*>(index_q);
   const auto* ik = static_cast<const uint16_t*>(index_k);
-  if (row_mask + 1 >= 64)
+  if (row_mask + 1 >= 64 && block_size % 64 == 0) {
+    hipLaunchKernelGGL((index_scores_rounds_kernel<128, 4>), dim3(block_stride, seq_len),
+                       dim3(64), 0, stream, image, iq, ik, scores, block_stride, block_size,
+                       scale, shift, row_mask);
+  } else if (row_mask + 1 >= 64)
     hipLaunchKernelGGL((index_scores_kernel<128, 4, true>), grid, dim3(256), 0,
                        stream, image, iq, ik, scores, block_stride, block_size, scale, shift,
                        row_mask);
