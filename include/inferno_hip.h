@@ -328,7 +328,9 @@ int32_t ifr_bq_block_sparse_attention(
  * weight [rows][cols], f32 accumulation.  rows % 16 == 0, cols % 128 == 0
  * (the reference also takes a scalar tail of cols % 32; not provided).  Small
  * seq_len splits the contraction over workgroups into f32 partials in
- * `workspace` (ifr_gemm_cols_workspace_bytes; 0 means none is needed). */
+ * `workspace` (ifr_gemm_cols_workspace_bytes; 0 means none is needed).  Past 64
+ * tokens a smaller workspace, or none where the output has more than 256 tiles of
+ * 64 x 64, runs with the splits that fit it. */
 int64_t ifr_gemm_cols_workspace_bytes(int64_t rows, int64_t cols, int64_t seq_len);
 int32_t ifr_dispatch_gemm_cols(const void* x, const void* weight, void* output,
                                int64_t rows, int64_t cols, int64_t seq_len,

@@ -1378,11 +1378,13 @@ int32_t ifr_dispatch_gemm_cols(const void* x, const void* weight, void* output, 
   if (!x || !weight || !output) return fail(IFR_EINVAL, "null pointer");
   if (!aligned(x, 16) || !aligned(weight, 16) || !aligned(output, 16))
     return fail(IFR_EINVAL, "x, weight and output must be 16-byte aligned");
-  const int64_t need = ifr::gemm_cols_workspace_bytes(seq_len, rows, cols);
-  if (need > 0 && (!workspace || workspace_bytes < need || !aligned(workspace, 16)))
+  const int64_t need = ifr::gemm_cols_required_bytes(seq_len, rows, cols);
+  const bool usable = workspace && aligned(workspace, 16);
+  if (need > 0 && (!usable || workspace_bytes < need))
     return fail(IFR_ESPACE, "workspace needs %lld bytes, 16-byte aligned", (long long)need);
-  IFR_HIP(ifr::launch_gemm_cols(x, weight, output, static_cast<float*>(workspace), seq_len,
-                                rows, cols, as_stream(stream)),
+  IFR_HIP(ifr::launch_gemm_cols(x, weight, output, static_cast<float*>(workspace),
+                                usable ? workspace_bytes : 0, seq_len, rows, cols,
+                                as_stream(stream)),
           "gemm_cols");
   return ok();
 }

@@ -404,13 +404,14 @@ hipError_t launch_tile(const uint16_t* x, const uint16_t* w, uint16_t* out, floa
 // k and the card runs 256 of them at a time (the 64 x 64 tile three per CU, so
 // its partial rounds cost their share only); splits add the reduce launch,
 // their own start and the f32 partials' way out and back.  It picks the
-// measured best or one within 5 % of it (12 % at 128 tokens): 128 x 128 in two
-// splits 21.8 us at 500 tokens, 192 x 128 45.1 us at 2,000 (242 of 256 CUs;
+// measured best or one within 5 % of it (12 % at 128 tokens): 128 x 64 22.2 us at
+// 500 tokens (two splits of 128 x 128 21.8), 192 x 128 45.1 us at 2,000 (242 of 256 CUs;
 // 256 x 128, 176 tiles, 47.9), 256 x 128 342 us at 16,384 (1,106 TFLOP/s).
+// Splits whose partials do not fit the caller's workspace are left out.
 struct TilePlan {
   int bm, bn, splits;
 };
-TilePlan tile_plan(int64_t M, int64_t N, int64_t K) {
+TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes) {
   struct Shape {
     int bm, bn;
     double us;
@@ -423,6 +424,7 @@ TilePlan tile_plan(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ((M + sh.bm - 1) / sh.bm) * ((N + sh.bn - 1) / sh.bn);
     for (int splits = 1; splits <= kMaxSplits; splits *= 2) {
       if ((K / 128) % splits != 0 || (splits > 1 && tiles * splits > 512)) break;
+      if (splits > 1 && splits * M * N * 4 > workspace_bytes) break;
       const double load = static_cast<double>(tiles * splits) / 256.0;
       const double rounds =
           sh.bm == 64 ? (load > 1.0 ? load : 1.0) : static_cast<double>((tiles * splits + 255) / 256);
@@ -449,29 +451,36 @@ hipError_t launch_plan(const TilePlan& p, const uint16_t* x, const uint16_t* w, 
 
 }  // namespace
 
-int gemm_cols_splits(int64_t M, int64_t N, int64_t K) {
-  const int span = decode_span(M, K);
-  if (span) return static_cast<int>(K / span);
-  return tile_plan(M, N, K).splits;
+int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (const int span = decode_span(M, K))
+    return M <= 16 ? 0 : K / span * M * N * 4;  // up to 16 tokens the slices meet in LDS
+  const int splits = tile_plan(M, N, K, INT64_MAX).splits;
+  return splits > 1 ? splits * M * N * 4 : 0;
 }
 
-int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  const int splits = gemm_cols_splits(M, N, K);
-  const bool sliced = decode_span(M, K) != 0;
-  if (sliced && M <= 16) return 0;  // the slices meet in LDS
-  return splits > 1 || sliced ? static_cast<int64_t>(splits) * M * N * 4 : 0;
+// Batches of more than 256 tiles of 64 x 64 run without a workspace, fewer with
+// room for two splits; what the plan takes beyond that is a matter of speed (400
+// tokens x 2816 x 8192: four splits 33.8 us, two 32.4, none 41.1).
+int64_t gemm_cols_required_bytes(int64_t M, int64_t N, int64_t K) {
+  const int64_t wanted = gemm_cols_workspace_bytes(M, N, K);
+  if (decode_span(M, K)) return wanted;
+  const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
+  return tiles > 256 ? 0 : std::min(wanted, 2 * M * N * 4);
 }
 
 hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* workspace,
-                            int64_t M, int64_t N, int64_t K, hipStream_t stream) {
+                            int64_t workspace_bytes, int64_t M, int64_t N, int64_t K,
+                            hipStream_t stream) {
   if (M <= 0) return hipSuccess;
-  const int splits = gemm_cols_splits(M, N, K);
+  const int span = decode_span(M, K);
+  const TilePlan plan = span ? TilePlan{} : tile_plan(M, N, K, workspace_bytes);
+  const int splits = span ? static_cast<int>(K / span) : plan.splits;
   const auto* xp = static_cast<const uint16_t*>(x);
   const auto* wp = static_cast<const uint16_t*>(w);
   auto* op = static_cast<uint16_t*>(out);
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
   hipError_t err;
-  if (const int span = decode_span(M, K)) {
+  if (span) {
     dim3 sgrid(static_cast<unsigned>((N + kBN - 1) / kBN), static_cast<unsigned>(splits));
     const int tm = static_cast<int>((M + 15) / 16);
     if (tm == 1) {
@@ -498,7 +507,7 @@ hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* work
     }
     err = hipGetLastError();
   } else {
-    err = launch_plan(tile_plan(M, N, K), xp, wp, op, workspace, m, n, k, stream);
+    err = launch_plan(plan, xp, wp, op, workspace, m, n, k, stream);
     if (splits == 1) return err;
   }
   if (err != hipSuccess) return err;

@@ -114,11 +114,14 @@ hipError_t launch_bq_block_quant(const void* src, void* x_i8, float* x_sa, int64
                                  int block, int64_t seq_len, hipStream_t stream);
 
 // dispatch_gemm_cols: out[m][n] = bf16(sum_k x[m][k] * w[n][k]); N % 16 == 0,
-// K % 128 == 0.  k splits (and with them the workspace) depend on the shape.
-int gemm_cols_splits(int64_t M, int64_t N, int64_t K);
+// K % 128 == 0.  k splits (and with them the workspace) depend on the shape and, past
+// the decode batches, on the workspace that there is: _workspace_bytes is what the
+// fastest plan uses, _required_bytes what the launch cannot do without.
 int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int64_t gemm_cols_required_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* workspace,
-                            int64_t M, int64_t N, int64_t K, hipStream_t stream);
+                            int64_t workspace_bytes, int64_t M, int64_t N, int64_t K,
+                            hipStream_t stream);
 
 // MiniMax-M3 lightning indexer (block scores + top-k) and block-sparse
 // attention over a full-attention plan image.

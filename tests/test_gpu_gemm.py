@@ -86,6 +86,27 @@ def test_gemm_cols_few_tokens_bit_exact(seq, rows, cols):
     test_gemm_cols_integer_operands_bit_exact(seq, rows, cols)
 
 
+@pytest.mark.parametrize("seq,splits", [(400, 0), (400, 1), (400, 2), (400, 3.99), (400, 4),
+                                        (321, 0), (200, 2), (200, 7)])
+def test_gemm_cols_workspace_smaller_than_the_plan(seq, splits):
+    """Room for that many splits' partials.  The plan takes four at these sizes; past
+    320 tokens (more than 256 tiles of 64 x 64) none are needed, before that two.
+    Integer operands, so every split count is exact."""
+    rows, cols = 2816, 8192
+    announce(f"gemm_cols workspace seq={seq} splits={splits}")
+    rng = np.random.default_rng(seq)
+    x = rng.integers(-3, 4, (seq, cols)).astype(np.float32)
+    w = rng.integers(-3, 4, (rows, cols)).astype(np.float32)
+    out = empty_dev(seq * rows, np.uint16)
+    floats = int(splits * seq * rows)
+    ws = to_dev(np.full(floats + 4096, 7.0, np.float32))  # the last 4,096 stay as they are
+    A.dispatch_gemm_cols(to_dev(_bf(x)), to_dev(_bf(w)), out, rows=rows, cols=cols, seq_len=seq,
+                         workspace=ws[:floats] if floats else None)
+    assert np.array_equal(from_dev(out, np.uint16).reshape(seq, rows),
+                          oracle.f32_to_bf16((x @ w.T).ravel()).reshape(seq, rows))
+    assert np.all(from_dev(ws, np.float32)[floats:] == 7.0)
+
+
 def test_gemm_cols_rejects_unsupported_shapes():
     from inferno_amd._lib import InfernoHipError
 
@@ -99,3 +120,6 @@ def test_gemm_cols_rejects_unsupported_shapes():
     assert A.gemm_cols_workspace(64, 512, 64) is not None  # this shape splits k
     with pytest.raises(InfernoHipError):
         A.dispatch_gemm_cols(x, w, out, rows=64, cols=512, seq_len=64)  # no workspace
+    x, w, out = (empty_dev(n, np.uint16) for n in (65 * 8192, 64 * 8192, 65 * 64))
+    with pytest.raises(InfernoHipError):
+        A.dispatch_gemm_cols(x, w, out, rows=64, cols=8192, seq_len=65)  # nor past the decode sizes
