@@ -57,7 +57,8 @@ __device__ __forceinline__ float groups_add(float x) {
 // the transposing LDS reads, which carry no alias information, and would wait
 // there for every load in flight.  The waits are written out below (loads return
 // in order, so the ones the compiler adds for its own loads can only wait for
-// more).  m0 is put back, as the compiler does not know of the change.
+// more).  m0 is put back, as the compiler does not know of the change; a write of m0
+// needs one wait state before a load that reads it.
 __device__ __forceinline__ uint32_t lds_addr(const uint8_t* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_t*)p));
 }
@@ -65,7 +66,7 @@ __device__ __forceinline__ void load_lds4(const char* base, uint32_t o0, uint32_
                                           uint32_t o3, const uint8_t* lds) {
   uint32_t m0;
   asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\t"
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
       "global_load_lds_dwordx4 %2, %6\n\t"
       "global_load_lds_dwordx4 %3, %6 offset:1024\n\t"
       "global_load_lds_dwordx4 %4, %6 offset:2048\n\t"
@@ -79,7 +80,7 @@ __device__ __forceinline__ void load_lds2(const char* base, uint32_t o0, uint32_
                                           const uint8_t* lds) {
   uint32_t m0;
   asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\t"
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
       "global_load_lds_dwordx4 %2, %4\n\t"
       "global_load_lds_dwordx4 %3, %4 offset:1024\n\t"
       "s_mov_b32 m0, %0"
