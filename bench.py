@@ -730,7 +730,7 @@ class SparseM3:
 
     dtype = "bf16 (indexer VDPBF16PS-order f32 dots; attention MFMA QK, f32 PV)"
     phases = ("indexer", "sparse")
-    dominant = "index_scores_kernel + select_blocks_kernel"
+    dominant = "index_scores_rounds_kernel + select_blocks_kernel"
     dominant_phase = "indexer"
     NQ, NKV, HD, IH, BLOCK, TOPK, PLEN = 64, 4, 128, 4, 128, 16, 128
 
@@ -954,7 +954,7 @@ class PrefillBf16:
                      "write), 16q/2kv hd512 bf16, partial RoPE (half 64, pair_stride 256)")
         else:
             self.nq, self.nkv, self.hd, self.half, self.pair = 16, 8, 256, 128, 128
-            self.dominant = "prefill_full_mfma_kernel"
+            self.dominant = "prefill_full_mfma_kernel" if self.bq else "prefill_pair_kernel"
             label = ("config4: chunked prefill, 8 sequences x 2048 new tokens on prefixes "
                      "~ U[0,16384] shared by sequence pairs (sealed pages shared, the partial "
                      "page copied on write), 16q/8kv hd256 bf16")

@@ -10,6 +10,8 @@
 //                       and forms the dots in the reference's VDPBF16PS order,
 //                       so block scores, and with them the selected blocks,
 //                       are bit-identical.
+// index_scores_rounds_kernel  the same with keys through LDS, for pages and index
+//                       blocks of whole 64-position rounds.
 // select_blocks_kernel  one wave per (token, index head): the reference's
 //                       32-slot streaming bank, each reduction done as a rank
 //                       count under reduce_argmax's order (value, then slot
