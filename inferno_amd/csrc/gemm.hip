@@ -129,7 +129,10 @@ void gemm_cols_tile_kernel(
   auto chunk = [&](int c, const uint8_t* cur, uint8_t* next) {
     // Chunk c has landed when only chunk c + 1's loads are outstanding.
     __builtin_amdgcn_s_waitcnt(0x0F70 | kLoads);  // vmcnt(kLoads)
-    asm volatile("s_barrier" ::: "memory");
+    // The reads of chunk c - 1 have returned before another wave may refill their
+    // buffer.  Written out: the compiler waits for them only where it puts the
+    // MFMAs that use them, which at 128 x 64 is partly behind the barrier.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // Past the last chunk the loads repeat it into a buffer nothing reads, so
     // the count of outstanding loads is the same in every iteration.
     const int cn = min(c + 2, nk - 1);
