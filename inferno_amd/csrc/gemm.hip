@@ -9,7 +9,8 @@
 // from HBM into registers.  They have too few output tiles to fill 256 CUs:
 // gemm_cols_split_kernel gives each workgroup a slice of k loaded in one round
 // trip and writes f32 partials that gemm_cols_reduce_kernel adds in slice
-// order; up to 16 tokens gemm_cols_few_kernel keeps the slices in one workgroup.
+// order; up to 16 tokens and k of 4,096 gemm_cols_few_kernel keeps the slices in one
+// workgroup.
 // Larger batches run gemm_cols_tile_kernel, LDS-tiled on
 // v_mfma_f32_32x32x16_bf16, in the tile shape and k splits of tile_plan.
 #include <algorithm>
@@ -292,19 +293,22 @@ __global__ __launch_bounds__(256) void gemm_cols_split_kernel(
   }
 }
 
-// At most 16 tokens: a workgroup takes up to 16 columns with one wave per k
-// slice, so the slices' partials meet in LDS instead of memory and there is no
-// reduce launch.  Each wave issues every load of its slice at once (x comes from
-// L2: at most 128 KiB, read by every workgroup); the partials are added in slice
-// order, so the bits are those of the split kernel and its reduce.
+// At most 16 tokens and k of up to 4,096: a workgroup takes up to 16 columns with
+// one wave per 256-wide k slice, so the slices' partials meet in LDS instead of
+// memory and there is no reduce launch.  Each wave issues every load of its slice
+// at once (x comes from L2: at most 128 KiB, read by every workgroup); the partials
+// are added in slice order, so the bits are those of the split kernel and its reduce.
 //
 // What bounds it is a memory round trip and each CU's share of w, so the columns
 // are spread over all 256 CUs (2,816: 11 a workgroup; lanes past them repeat the
 // last).  Plain loads: a fragment load takes half of each 128-byte line, the next
 // one the other half.  One token x 2816 x 4096 from HBM, launches back to back:
 // split kernel and reduce 9.0 us, 16 columns with non-temporal loads 8.0, with
-// plain ones 7.6, 11 columns 7.0; 16 tokens 10.6 -> 9.2.
-template <int kSpan>
+// plain ones 7.6, 11 columns 7.0; 16 tokens 10.6 -> 9.2.  Slices of 512, which k of
+// 8,192 would take, hold 128 registers of operands where 16 waves leave 128 in all:
+// 2816 x 8192 13.1 -> 13.3 us at one token and 14.5 -> 18.0 at 16, so they stay with
+// the split kernel.
+constexpr int kFewSpan = 256;
 __global__ __launch_bounds__(64 * kMaxSplits) void gemm_cols_few_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, uint16_t* __restrict__ out,
     int M, int N, int K, int cols) {
@@ -314,25 +318,25 @@ __global__ __launch_bounds__(64 * kMaxSplits) void gemm_cols_few_kernel(
   const int r = lane & 15;
   const int g = lane >> 4;
   const int n0 = blockIdx.x * cols;
-  const int k0 = wave * kSpan + 8 * g;
+  const int k0 = wave * kFewSpan + 8 * g;
   const int n = min(n0 + min(r, cols - 1), N - 1);
   const uint16_t* wp = w + static_cast<int64_t>(n) * K + k0;
   const uint16_t* xp = x + static_cast<int64_t>(min(r, M - 1)) * K + k0;
-  uint4 wr[kSpan / 32], xr[kSpan / 32];
+  uint4 wr[kFewSpan / 32], xr[kFewSpan / 32];
 #pragma unroll
-  for (int j = 0; j < kSpan / 32; ++j) wr[j] = *reinterpret_cast<const uint4*>(wp + 32 * j);
+  for (int j = 0; j < kFewSpan / 32; ++j) wr[j] = *reinterpret_cast<const uint4*>(wp + 32 * j);
 #pragma unroll
-  for (int j = 0; j < kSpan / 32; ++j) xr[j] = *reinterpret_cast<const uint4*>(xp + 32 * j);
+  for (int j = 0; j < kFewSpan / 32; ++j) xr[j] = *reinterpret_cast<const uint4*>(xp + 32 * j);
   __builtin_amdgcn_sched_barrier(0);  // every load ahead of the first MFMA
   f32x4_t acc{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int j = 0; j < kSpan / 32; ++j)
+  for (int j = 0; j < kFewSpan / 32; ++j)
     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xr[j]),
                                                   __builtin_bit_cast(bf16x8_t, wr[j]), acc, 0, 0, 0);
 #pragma unroll
   for (int j = 0; j < 4; ++j) part[wave][4 * g + j][r] = acc[j];
   __syncthreads();
-  const int slices = K / kSpan;
+  const int slices = K / kFewSpan;
   for (int i = threadIdx.x; i < cols * M; i += blockDim.x) {
     const int m = i / cols, c = i - m * cols;
     if (n0 + c >= N) continue;
@@ -381,7 +385,7 @@ hipError_t launch_reduce_n(const float* part, uint16_t* out, int64_t quads, int6
 
 // k slice of the decode kernels, or 0 when the batch takes the tile kernel.
 int decode_span(int64_t M, int64_t K) {
-  if (M <= 16 && K % 256 == 0 && K / 256 <= kMaxSplits) return 256;
+  if (M <= 16 && K % kFewSpan == 0 && K / kFewSpan <= kMaxSplits) return kFewSpan;
   if (M <= kBM && K % 512 == 0 && K / 512 <= kMaxSplits) return 512;
   return 0;
 }
@@ -456,7 +460,7 @@ hipError_t launch_plan(const TilePlan& p, const uint16_t* x, const uint16_t* w, 
 
 int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (const int span = decode_span(M, K))
-    return M <= 16 ? 0 : K / span * M * N * 4;  // up to 16 tokens the slices meet in LDS
+    return span == kFewSpan ? 0 : K / span * M * N * 4;  // there the slices meet in LDS
   const int splits = tile_plan(M, N, K, INT64_MAX).splits;
   return splits > 1 ? splits * M * N * 4 : 0;
 }
@@ -486,19 +490,17 @@ hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* work
   if (span) {
     dim3 sgrid(static_cast<unsigned>((N + kBN - 1) / kBN), static_cast<unsigned>(splits));
     const int tm = static_cast<int>((M + 15) / 16);
-    if (tm == 1) {
+    if (span == kFewSpan) {
       const int cols = static_cast<int>(std::min<int64_t>(16, (N + 255) / 256));
       const dim3 fgrid(static_cast<unsigned>((N + cols - 1) / cols));
-      const dim3 block(static_cast<unsigned>(64 * splits));
-      if (span == 256)
-        hipLaunchKernelGGL(gemm_cols_few_kernel<256>, fgrid, block, 0, stream, xp, wp, op, m, n, k,
-                           cols);
-      else
-        hipLaunchKernelGGL(gemm_cols_few_kernel<512>, fgrid, block, 0, stream, xp, wp, op, m, n, k,
-                           cols);
+      hipLaunchKernelGGL(gemm_cols_few_kernel, fgrid, dim3(static_cast<unsigned>(64 * splits)), 0,
+                         stream, xp, wp, op, m, n, k, cols);
       return hipGetLastError();
     }
-    if (tm == 2) {
+    if (tm == 1) {
+      hipLaunchKernelGGL((gemm_cols_split_kernel<1, 512>), sgrid, dim3(256), 0, stream, xp,
+                         wp, workspace, m, n, k);
+    } else if (tm == 2) {
       hipLaunchKernelGGL((gemm_cols_split_kernel<2, 512>), sgrid, dim3(256), 0, stream, xp,
                          wp, workspace, m, n, k);
     } else if (tm == 3) {

@@ -1,4 +1,5 @@
-"""The workgroup barriers of the kernels that write their own (inline `s_barrier`
+"""What the kernels' own waits and launch bounds rest on, in the gfx950 code that the
+compiler makes of them.  The workgroup barriers of the kernels that write their own (inline `s_barrier`
 instead of __syncthreads, so that loads in flight stay in flight), in the gfx950
 code that the compiler makes of them: on every path, no LDS access of the wave may
 still be outstanding when it arrives.  Another wave may overwrite that LDS right
@@ -72,17 +73,27 @@ def test_the_scan_sees_reads_behind_waits_and_round_loops():
     assert outstanding_at_barriers(loop) == (1, [("s_barrier", 16)])
 
 
-@pytest.mark.parametrize("source", OWN_BARRIERS)
-def test_no_lds_access_outstanding_at_a_barrier(source, tmp_path):
+def _device_code(source, tmp_path):
     asm = tmp_path / "device.s"
     res = subprocess.run([hipcc(), *COMMON_FLAGS, "--cuda-device-only", "-S", str(CSRC / source),
                           "-o", str(asm)], capture_output=True, text=True)
     assert res.returncode == 0, res.stderr
+    return asm.read_text()
+
+
+@pytest.mark.parametrize("source", OWN_BARRIERS)
+def test_no_lds_access_outstanding_at_a_barrier(source, tmp_path):
     barriers, faults = 0, {}
-    for name, lines in _functions(asm.read_text()).items():
+    for name, lines in _functions(_device_code(source, tmp_path)).items():
         n, late = outstanding_at_barriers(lines)
         barriers += n
         if late:
             faults[name] = late
     assert barriers > 0
     assert not faults, faults
+
+
+def test_gemm_kernels_keep_their_operands_in_registers(tmp_path):
+    asm = _device_code("gemm.hip", tmp_path)
+    sizes = re.findall(r"\.amdhsa_kernel (\S+).*?\.amdhsa_private_segment_fixed_size (\d+)", asm, re.S)
+    assert sizes and all(int(n) == 0 for _, n in sizes), [k for k, n in sizes if int(n)]

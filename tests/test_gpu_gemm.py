@@ -79,10 +79,11 @@ def test_gemm_cols_tiles_bit_exact(seq, rows, cols):
 
 
 @pytest.mark.parametrize("seq,rows,cols", [(1, 16, 256), (1, 2816, 4096), (15, 48, 512),
-                                           (16, 2816, 8192), (7, 80, 1536), (17, 80, 4096)])
+                                           (16, 2816, 8192), (1, 80, 8192), (11, 48, 4608),
+                                           (7, 80, 1536), (17, 80, 4096)])
 def test_gemm_cols_few_tokens_bit_exact(seq, rows, cols):
-    """One to sixteen tokens (slices joined in the workgroup) and the first
-    size past them, 1 to 16 slices of 256 and 512."""
+    """One to sixteen tokens and the first size past them: 1 to 16 slices of 256
+    (joined in the workgroup) and, past k of 4,096 or 16 tokens, of 512."""
     test_gemm_cols_integer_operands_bit_exact(seq, rows, cols)
 
 
@@ -121,5 +122,7 @@ def test_gemm_cols_rejects_unsupported_shapes():
     with pytest.raises(InfernoHipError):
         A.dispatch_gemm_cols(x, w, out, rows=64, cols=512, seq_len=64)  # no workspace
     x, w, out = (empty_dev(n, np.uint16) for n in (65 * 8192, 64 * 8192, 65 * 64))
+    with pytest.raises(InfernoHipError):
+        A.dispatch_gemm_cols(x, w, out, rows=64, cols=8192, seq_len=16)
     with pytest.raises(InfernoHipError):
         A.dispatch_gemm_cols(x, w, out, rows=64, cols=8192, seq_len=65)  # nor past the decode sizes
