@@ -700,25 +700,52 @@ int32_t ifr_rms_norm_rope_cache_write(const void* image_dev, const int64_t* info
 }  // extern "C"
 
 namespace {
-// Which MFMA prefill kernel, if any, runs a bf16 plan: token plans with
-// query blocks at the shapes the kernels are built for (full attention at
-// head_dim 256 / GQA 2 and 512 / GQA 8, sliding windows at 256 / GQA 2).
-enum class PrefillRoute { kNone, kFull256, kWide512, kSliding256 };
-PrefillRoute bf16_prefill_route(const int64_t* info, int64_t num_q, int64_t num_kv,
-                                int64_t head_dim, int64_t page_mask) {
-  if (info[14] <= 0) return PrefillRoute::kNone;
-  if (info[2] == IFR_PLAN_TOKEN_MERGE && page_mask < 0) {
-    if (head_dim == 256 && num_q == 2 * num_kv) return PrefillRoute::kFull256;
-    if (head_dim == 512 && num_q == 8 * num_kv) return PrefillRoute::kWide512;
+// The kernel of a bf16 plan.  The MFMA prefill kernels take token plans with query
+// blocks at the shapes they are built for: full attention at head_dim 256 / GQA 2 and
+// 512 / GQA 8, sliding windows at 256 / GQA 2.
+enum Bf16Route {
+  kRoutePartials,     // partials and merge, or one item per token
+  kRouteNarrowTiles,  // prefill_narrow_tiles_kernel
+  kRouteNarrowPairs,  // prefill_narrow_pairs_kernel
+  kRoutePair,         // prefill_pair_kernel
+  kRouteFull,         // prefill_full_mfma_kernel
+  kRouteWide,         // prefill_wide_mfma_kernel
+  kRouteSliding,      // prefill_sliding_mfma_kernel
+};
+Bf16Route bf16_route(const int64_t* info, int64_t num_q, int64_t num_kv, int64_t head_dim,
+                     int64_t kv_stride, int64_t page_mask) {
+  if (info[14] <= 0) return kRoutePartials;
+  const int shift = static_cast<int>(info[7]);
+  if (info[2] == IFR_PLAN_TOKEN_MERGE && page_mask < 0 &&
+      ((head_dim == 256 && num_q == 2 * num_kv) || (head_dim == 512 && num_q == 8 * num_kv))) {
+    const int kind = ifr::prefill_narrow_kind(info[14], info[6], info[5], num_kv,
+                                              static_cast<int>(head_dim), kv_stride, shift);
+    if (kind) return kind == 2 ? kRouteNarrowPairs : kRouteNarrowTiles;
+    if (head_dim == 512) return kRouteWide;
+    return ifr::prefill_pair_takes(kv_stride, shift) ? kRoutePair : kRouteFull;
   }
   if (info[2] == IFR_PLAN_TOKEN_DIRECT && page_mask >= 0 && head_dim == 256 &&
       num_q == 2 * num_kv)
-    return PrefillRoute::kSliding256;
-  return PrefillRoute::kNone;
+    return kRouteSliding;
+  return kRoutePartials;
 }
 }  // namespace
 
 extern "C" {
+
+// Not part of the C API: the route (its number above) and, for the narrow kernels,
+// the workgroups of ifr_attention_bf16, for the tests to hold on to.
+int32_t ifr_internal_bf16_route(const int64_t* info, int64_t num_q, int64_t num_kv,
+                                int64_t head_dim, int64_t kv_stride, int64_t* route) {
+  int32_t st = check_info(info);
+  if (st) return st;
+  route[0] = bf16_route(info, num_q, num_kv, head_dim, kv_stride, info[9]);
+  route[1] = route[0] == kRouteNarrowTiles || route[0] == kRouteNarrowPairs
+                 ? ifr::prefill_narrow_blocks(info[14], info[6], info[5], num_kv,
+                                              static_cast<int>(head_dim))
+                 : 0;
+  return ok();
+}
 
 int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
                            const void* q, const void* k_base,
@@ -742,35 +769,33 @@ int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
   if (st) return st;
   ifr::PagedGeom g{static_cast<int>(pow2_shift(page_len)), static_cast<int>(page_len - 1),
                    static_cast<int>(page_mask)};
-  const PrefillRoute route = bf16_prefill_route(info, num_q, num_kv, head_dim, page_mask);
+  const Bf16Route route = bf16_route(info, num_q, num_kv, head_dim, kv_stride, page_mask);
   // The MFMA prefill routes finalise in-kernel and write no partials.
-  if (route == PrefillRoute::kNone && partials_bytes < info[3] * partial_stride * 4)
+  if (route == kRoutePartials && partials_bytes < info[3] * partial_stride * 4)
     return fail(IFR_ESPACE, "partials need %lld bytes", (long long)(info[3] * partial_stride * 4));
-  if (route == PrefillRoute::kFull256 || route == PrefillRoute::kWide512) {
-    const int kind =
-        ifr::prefill_narrow_kind(info[14], info[6], info[5], num_kv, static_cast<int>(head_dim),
-                                 kv_stride, static_cast<int>(pow2_shift(page_len)));
-    if (kind) {
-      // Few rows (a short chunk, or tokens decoding beside one).
-      IFR_HIP(ifr::launch_prefill_narrow(static_cast<const int32_t*>(image_dev), kind,
-                                         static_cast<int>(info[14]), q, k_base, v_base, output,
-                                         static_cast<int>(head_dim), static_cast<int>(num_q),
-                                         static_cast<int>(num_kv), kv_stride, g,
-                                         as_stream(stream)),
-              "prefill_narrow");
-      return ok();
-    }
-  }
-  if (route == PrefillRoute::kFull256) {
-    // Prefill chunk of full attention: MFMA query blocks, finalised in-kernel.
-    if (ifr::prefill_pair_takes(kv_stride, static_cast<int>(pow2_shift(page_len)))) {
-      IFR_HIP(ifr::launch_prefill_pair(static_cast<const int32_t*>(image_dev),
-                                       static_cast<int>(info[14]), q, k_base, v_base, output,
+  if (route == kRouteNarrowTiles || route == kRouteNarrowPairs) {
+    // Few rows (a short chunk, or tokens decoding beside one).
+    const int64_t blocks = ifr::prefill_narrow_blocks(info[14], info[6], info[5], num_kv,
+                                                      static_cast<int>(head_dim));
+    IFR_HIP(ifr::launch_prefill_narrow(static_cast<const int32_t*>(image_dev),
+                                       route == kRouteNarrowPairs ? 2 : 1, blocks, q,
+                                       k_base, v_base, output, static_cast<int>(head_dim),
                                        static_cast<int>(num_q), static_cast<int>(num_kv),
                                        kv_stride, g, as_stream(stream)),
-              "prefill_pair");
-      return ok();
-    }
+            "prefill_narrow");
+    return ok();
+  }
+  if (route == kRoutePair) {
+    // Prefill chunk of full attention: MFMA query blocks, finalised in-kernel.
+    IFR_HIP(ifr::launch_prefill_pair(static_cast<const int32_t*>(image_dev),
+                                     static_cast<int>(info[14]), q, k_base, v_base, output,
+                                     static_cast<int>(num_q), static_cast<int>(num_kv),
+                                     kv_stride, g, as_stream(stream)),
+            "prefill_pair");
+    return ok();
+  }
+  if (route == kRouteFull) {
+    // The same over pages of fewer than 16 rows.
     IFR_HIP(ifr::launch_prefill_full_mfma(static_cast<const int32_t*>(image_dev),
                                           static_cast<int>(info[14]), q, k_base, v_base,
                                           output, static_cast<int>(num_q),
@@ -779,7 +804,7 @@ int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
             "prefill_full_mfma");
     return ok();
   }
-  if (route == PrefillRoute::kWide512) {
+  if (route == kRouteWide) {
     // The same at Gemma-4's full-attention shape (head_dim 512, GQA 8).
     IFR_HIP(ifr::launch_prefill_wide_mfma(static_cast<const int32_t*>(image_dev),
                                           static_cast<int>(info[14]), q, k_base, v_base,
@@ -789,7 +814,7 @@ int32_t ifr_attention_bf16(const void* image_dev, const int64_t* info,
             "prefill_wide_mfma");
     return ok();
   }
-  if (route == PrefillRoute::kSliding256) {
+  if (route == kRouteSliding) {
     // Prefill chunk of a sliding-window layer: MFMA query blocks.
     IFR_HIP(ifr::launch_prefill_sliding_mfma(static_cast<const int32_t*>(image_dev),
                                              static_cast<int>(info[14]), q, k_base, v_base,
@@ -855,8 +880,8 @@ int32_t ifr_attention_bf16_noalloc(const void* image_dev, const int64_t* info, c
     return fail(IFR_EINVAL, "bad num_q or head_dim");
   const int64_t ps = ifr_flash_partial_stride(num_q, head_dim);
   // The MFMA prefill routes write no partials, so their chunks need no scratch.
-  const bool mfma = bf16_prefill_route(info, num_q, num_kv, head_dim, page_mask) !=
-                    PrefillRoute::kNone;
+  const bool mfma =
+      bf16_route(info, num_q, num_kv, head_dim, kv_stride, page_mask) != kRoutePartials;
   const int64_t need = mfma ? 0 : info[3] * ps * 4;
   if (need > kStaticScratchBytes)
     return fail(IFR_ESPACE,

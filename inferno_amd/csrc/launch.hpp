@@ -55,11 +55,13 @@ bool prefill_pair_takes(int64_t kv_stride, int page_shift);
 hipError_t launch_prefill_pair(const int32_t* image, int num_qblocks, const void* q,
                                const void* k, const void* v, void* output, int num_q, int num_kv,
                                int64_t kv_stride, PagedGeom geom, hipStream_t stream);
-// Full-attention prefill of few rows: the kernel for a plan (0: none of these),
-// and its launch.
+// Full-attention prefill of few rows: the blocks that a launch needs, the kernel for a
+// plan (0: none of these), and its launch.
+int64_t prefill_narrow_blocks(int64_t num_qblocks, int64_t num_runs, int64_t seq_len,
+                              int64_t num_kv, int head_dim);
 int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, int64_t num_kv,
                         int head_dim, int64_t kv_stride, int page_shift);
-hipError_t launch_prefill_narrow(const int32_t* image, int kind, int num_qblocks, const void* q,
+hipError_t launch_prefill_narrow(const int32_t* image, int kind, int64_t blocks, const void* q,
                                  const void* k, const void* v, void* output, int head_dim,
                                  int num_q, int num_kv, int64_t kv_stride, PagedGeom geom,
                                  hipStream_t stream);

@@ -36,6 +36,7 @@
 // chunk 278 / 191 / 157; 374.  At 16 / 2 x 512
 // (query-block kernel / tiles): 64 tokens 518 / 275; 500 690 / 300; 1,000 750 /
 // 580; 2,000 671 / 1,230; the mixed step 630 / 290.
+#include <algorithm>
 #include <type_traits>
 
 #include "launch.hpp"
@@ -56,7 +57,8 @@ constexpr int kNW = 4;            // waves of a block
 // The sub-block (kTok tokens of a plan query block) that block number `rest`
 // takes, counting only those with tokens, in plan order and the longest key
 // range of a query block first: qb (-1 past the last) and sub.  The blocks
-// without one then all come last.  (A grid of every query block's sub-blocks in
+// without one then all come last, and the launch leaves them out but for a few
+// (prefill_narrow_blocks).  (A grid of every query block's sub-blocks in
 // order puts the single live one of each decoding token's query block on the
 // same shader engine: 64 of 256 CUs did that work.)
 template <int kTok>
@@ -934,12 +936,23 @@ void prefill_narrow_pairs_kernel(const int32_t* __restrict__ image, const uint16
 
 }  // namespace
 
+// Blocks of 32 rows (kTok tokens of a run, one kv head) that a launch needs: at most
+// this many have tokens, as every run may end in a partial one.  Of every query
+// block's 64 / kTok, most have none where many sequences decode, and each of those
+// walks the whole plan to find that out: 2,000 sequences of up to 100 keys beside 32
+// tokens 1,986 -> 271 us at 16 / 2 heads x 512, 1,065 -> 408 at 16 / 8 x 256.
+int64_t prefill_narrow_blocks(int64_t num_qblocks, int64_t num_runs, int64_t seq_len,
+                              int64_t num_kv, int head_dim) {
+  const int64_t tok = head_dim == 256 ? 16 : 4;
+  return std::min((seq_len + (tok - 1) * num_runs) / tok, kPrefillTokens / tok * num_qblocks) *
+         num_kv;
+}
+
 // Which kernel takes a full-attention token plan: 0 the query-block kernel, 1
 // tiles, 2 pairs.  A cost in us per 128 keys, from the measurements above: a
-// launch takes its 256 (or, tiles at head_dim 256, 512) blocks at a time.
-// live: blocks of 32 rows with tokens (an upper bound: every run may end in a
-// partial one).  The query-block kernels' later rounds overlap, so beyond one
-// round they cost their share of it.
+// launch takes its 256 (or, tiles at head_dim 256, 512) blocks at a time.  The
+// query-block kernels' later rounds overlap, so beyond one round they cost their
+// share of it.
 int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, int64_t num_kv,
                         int head_dim, int64_t kv_stride, int page_shift) {
   // Pages hold whole tiles, and a tile's row offsets fit 32 bits.
@@ -950,39 +963,38 @@ int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, 
   auto block_cost = [](int64_t blocks, double one, double more) {
     return blocks <= 256 ? one : (one > more * blocks / 256.0 ? one : more * blocks / 256.0);
   };
+  const int64_t live = prefill_narrow_blocks(num_qblocks, num_runs, seq_len, num_kv, head_dim);
   if (head_dim == 256) {
-    const int64_t live = (seq_len + 15 * num_runs) / 16 * num_kv;
     const double block = block_cost(num_qblocks * num_kv, 5.1, 6.3);
     const double pairs = 2.45 * rounds(live, 256);
     const double tiles = live <= 256 ? 3.2 : 4.3 * rounds(live, 512);
     if (block <= pairs && block <= tiles) return 0;
     return pairs <= tiles ? 2 : 1;
   }
-  const int64_t live = (seq_len + 3 * num_runs) / 4 * num_kv;
   return 5.05 * rounds(live, 256) < block_cost(4 * num_qblocks * num_kv, 11.5, 9.8) ? 1 : 0;
 }
 
-hipError_t launch_prefill_narrow(const int32_t* image, int kind, int num_qblocks, const void* q,
+hipError_t launch_prefill_narrow(const int32_t* image, int kind, int64_t blocks, const void* q,
                                  const void* k, const void* v, void* output, int head_dim,
                                  int num_q, int num_kv, int64_t kv_stride, PagedGeom geom,
                                  hipStream_t stream) {
-  if (num_qblocks <= 0) return hipSuccess;
+  if (blocks <= 0) return hipSuccess;
+  const dim3 grid(static_cast<unsigned>(blocks));
   const auto* qp = static_cast<const uint16_t*>(q);
   const auto* kp = static_cast<const uint16_t*>(k);
   const auto* vp = static_cast<const uint16_t*>(v);
   auto* op = static_cast<uint16_t*>(output);
-  const unsigned blocks = static_cast<unsigned>(num_qblocks) * static_cast<unsigned>(num_kv);
   if (head_dim == 256 && kind == 2)
-    hipLaunchKernelGGL((prefill_narrow_pairs_kernel<256, 2>), dim3(blocks * 4), dim3(64 * kNW), 0,
-                       stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+    hipLaunchKernelGGL((prefill_narrow_pairs_kernel<256, 2>), grid, dim3(64 * kNW), 0, stream,
+                       image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
                        geom.row_mask);
   else if (head_dim == 256)
-    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<256, 2, 2>), dim3(blocks * 4), dim3(64 * kNW),
-                       0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<256, 2, 2>), grid, dim3(64 * kNW), 0, stream,
+                       image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
                        geom.row_mask);
   else
-    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<512, 8, 1>), dim3(blocks * 16), dim3(64 * kNW),
-                       0, stream, image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
+    hipLaunchKernelGGL((prefill_narrow_tiles_kernel<512, 8, 1>), grid, dim3(64 * kNW), 0, stream,
+                       image, qp, kp, vp, op, num_q, num_kv, kv_stride, geom.shift,
                        geom.row_mask);
   return hipGetLastError();
 }

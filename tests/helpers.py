@@ -152,3 +152,21 @@ def seeded_bf16(n: int, seed: int) -> np.ndarray:
     f = rng.standard_normal(n).astype(np.float32)
     u = f.view(np.uint32).astype(np.uint64)
     return ((u + ((u >> 16) & 1) + 0x7FFF) >> 16).astype(np.uint16)
+
+
+# The kernels of ifr_attention_bf16, by the number that its route query gives them.
+(ROUTE_PARTIALS, ROUTE_NARROW_TILES, ROUTE_NARROW_PAIRS, ROUTE_PAIR, ROUTE_FULL, ROUTE_WIDE,
+ ROUTE_SLIDING) = range(7)
+
+
+def bf16_route(plan, num_q: int, num_kv: int, head_dim: int, kv_stride: int | None = None):
+    """(kernel, 32-row workgroups of the narrow kernels) that ifr_attention_bf16 launches."""
+    import ctypes as C
+
+    from inferno_amd._lib import I64, P_I64, check, lib
+
+    fn = lib().ifr_internal_bf16_route
+    fn.restype, fn.argtypes = C.c_int32, [P_I64, I64, I64, I64, I64, P_I64]
+    route = (C.c_int64 * 2)()
+    check(fn(plan.info_ptr, num_q, num_kv, head_dim, kv_stride or num_kv * head_dim, route))
+    return int(route[0]), int(route[1])

@@ -1,0 +1,53 @@
+"""Which kernel a full-attention token plan takes, and with how many workgroups
+(host rules; no GPU is touched)."""
+import numpy as np
+import pytest
+
+from inferno_amd.kv import FULL, AttentionPlan, KVRunTable
+from tests.helpers import (ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, bf16_route, make_prefill_case)
+
+
+def token_plan(prefix, new, page_len=64, num_kv=8, head_dim=256):
+    case = make_prefill_case(1, prefix, new, page_len=page_len)
+    table = KVRunTable()
+    for r in case.runs:
+        table.begin_run(int(r[0]), int(r[1]))
+        for j in range(int(r[3])):
+            table.add_base_row(int(case.base_rows[int(r[2]) + j]))
+    return AttentionPlan(table, sum(new), kind=FULL, window=0, cache_size=page_len,
+                         page_len=page_len, cache_rows=case.cache_rows, cap=1,
+                         kv_row_bytes=num_kv * head_dim * 2, device="cpu")
+
+
+def live_blocks(new, num_kv, tokens):
+    return num_kv * sum(-(-n // tokens) for n in new)
+
+
+@pytest.mark.parametrize("head_dim,num_kv,gqa,tokens", [(256, 8, 2, 16), (256, 1, 2, 16),
+                                                        (512, 2, 8, 4), (512, 1, 8, 4)])
+def test_narrow_workgroups_are_those_with_tokens(head_dim, num_kv, gqa, tokens):
+    """A workgroup without tokens looks for some through the whole plan: of many
+    sequences of one token each, there may be none."""
+    new = [1] * 500 + [32]
+    plan = token_plan([30] * 501, new, num_kv=num_kv, head_dim=head_dim)
+    kernel, blocks = bf16_route(plan, num_kv * gqa, num_kv, head_dim)
+    assert kernel in (ROUTE_NARROW_TILES, ROUTE_NARROW_PAIRS)
+    assert blocks == live_blocks(new, num_kv, tokens)
+
+
+@pytest.mark.parametrize("head_dim,num_kv,gqa,tokens", [(256, 8, 2, 16), (512, 2, 8, 4)])
+def test_narrow_workgroups_cover_every_token(head_dim, num_kv, gqa, tokens):
+    rng = np.random.default_rng(head_dim)
+    seen = 0
+    for _ in range(60):
+        n = int(rng.integers(1, 40))
+        new = [int(x) for x in np.ceil(2.0 ** rng.uniform(0, 7, n))]
+        kernel, blocks = bf16_route(token_plan([5] * n, new, num_kv=num_kv, head_dim=head_dim),
+                                    num_kv * gqa, num_kv, head_dim)
+        if kernel not in (ROUTE_NARROW_TILES, ROUTE_NARROW_PAIRS):
+            continue
+        seen += 1
+        live = live_blocks(new, num_kv, tokens)
+        # Every run may end in a partial block; no more than that is added.
+        assert live <= blocks <= live + num_kv * n
+    assert seen > 20
