@@ -968,7 +968,10 @@ int prefill_narrow_kind(int64_t num_qblocks, int64_t num_runs, int64_t seq_len, 
     const double block = block_cost(num_qblocks * num_kv, 5.1, 6.3);
     const double pairs = 2.45 * rounds(live, 256);
     const double tiles = live <= 256 ? 3.2 : 4.3 * rounds(live, 512);
-    if (block <= pairs && block <= tiles) return 0;
+    // Within 3 % the query-block kernel: what the costs leave out, a block's own start,
+    // is paid by more blocks in the narrow ones (300 runs of 20 tokens on up to 50 at
+    // one kv head, 7.38 against 7.35: pairs 25.7 us, prefill_pair_kernel 19.1).
+    if (block <= 1.03 * std::min(pairs, tiles)) return 0;
     return pairs <= tiles ? 2 : 1;
   }
   return 5.05 * rounds(live, 256) < block_cost(4 * num_qblocks * num_kv, 11.5, 9.8) ? 1 : 0;

@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 from inferno_amd.kv import FULL, AttentionPlan, KVRunTable
-from tests.helpers import (ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, bf16_route, make_prefill_case)
+from tests.helpers import (ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, ROUTE_PAIR, bf16_route,
+                           make_prefill_case)
 
 
 def token_plan(prefix, new, page_len=64, num_kv=8, head_dim=256):
@@ -51,3 +52,8 @@ def test_narrow_workgroups_cover_every_token(head_dim, num_kv, gqa, tokens):
         # Every run may end in a partial block; no more than that is added.
         assert live <= blocks <= live + num_kv * n
     assert seen > 20
+
+
+def test_a_tie_goes_to_the_query_blocks():
+    plan = token_plan([25] * 300, [20] * 300, num_kv=1)
+    assert bf16_route(plan, 2, 1, 256) == (ROUTE_PAIR, 0)
