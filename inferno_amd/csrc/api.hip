@@ -1238,6 +1238,11 @@ int64_t ifr_index_scores_bytes(const int64_t* info, int64_t num_index_heads,
   return info[5] * num_index_heads * ifr::index_block_stride(info[13], block_size) * 4;
 }
 
+// Not part of the C API, for the tests: the index blocks of a token that get a wave.
+int64_t ifr_internal_index_blocks(const int64_t* info, int64_t block_size) {
+  return ifr::index_blocks(info[13], block_size);
+}
+
 int32_t ifr_lightning_indexer(const void* image_dev, const int64_t* info, const void* index_q,
                               const void* index_k, int32_t* block_idx, float* scores,
                               int64_t scores_bytes, int64_t num_index_heads,
@@ -1267,9 +1272,10 @@ int32_t ifr_lightning_indexer(const void* image_dev, const int64_t* info, const 
     return fail(IFR_ESPACE, "scores need %lld bytes", (long long)need);
   IFR_HIP(ifr::launch_lightning_indexer(
               static_cast<const int32_t*>(image_dev), static_cast<int>(info[5]), index_q,
-              index_k, block_idx, scores, static_cast<int>(stride),
-              static_cast<int>(num_index_heads), static_cast<int>(index_head_dim),
-              static_cast<int>(block_size), static_cast<int>(topk_blocks),
+              index_k, block_idx, scores, ifr::index_blocks(info[13], block_size),
+              static_cast<int>(stride), static_cast<int>(num_index_heads),
+              static_cast<int>(index_head_dim), static_cast<int>(block_size),
+              static_cast<int>(topk_blocks),
               static_cast<int>(local_blocks), static_cast<int>(init_blocks), scale,
               static_cast<int>(info[7]), static_cast<int>(info[8]), as_stream(stream)),
           "lightning_indexer");

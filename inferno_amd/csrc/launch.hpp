@@ -127,12 +127,13 @@ hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* work
 
 // MiniMax-M3 lightning indexer (block scores + top-k) and block-sparse
 // attention over a full-attention plan image.
+int index_blocks(int64_t max_pos, int64_t block_size);  // of the longest context
 int index_block_stride(int64_t max_pos, int64_t block_size);
 int select_bank_cap(int topk);
 hipError_t launch_lightning_indexer(const int32_t* image, int seq_len, const void* index_q,
                                     const void* index_k, int32_t* block_idx, float* scores,
-                                    int block_stride, int num_heads, int head_dim,
-                                    int block_size, int topk, int local_blocks,
+                                    int num_blocks, int block_stride, int num_heads,
+                                    int head_dim, int block_size, int topk, int local_blocks,
                                     int init_blocks, float scale, int shift, int row_mask,
                                     hipStream_t stream);
 hipError_t launch_block_sparse_attention(const int32_t* image, int seq_len, const void* q,

@@ -200,7 +200,8 @@ __global__ __launch_bounds__(256) void index_scores_kernel(
 // by HBM where they do not.  Measured against index_scores_kernel, with the
 // selection: 64 tokens on 1,024 to 131,071 keys 242 -> 216 us, 16 on up to 60,000
 // 51 -> 46, one on 30,000 29.4 -> 26.4, 512 tokens of one sequence on 20,000
-// 380 -> 263.  Four waves a SIMD (12 fewer registers than needed) 287 us, several
+// 380 -> 263; 256 on up to 200 beside one on 100,000, nearly all waves without a
+// block, 70 -> 73.  Four waves a SIMD (12 fewer registers than needed) 287 us, several
 // blocks a wave 224 to 253.
 template <int D, int H>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3)))
@@ -1248,8 +1249,12 @@ tiles_done:
 
 }  // namespace
 
+int index_blocks(int64_t max_pos, int64_t block_size) {
+  return static_cast<int>(max_pos / block_size + 1);
+}
+
 int index_block_stride(int64_t max_pos, int64_t block_size) {
-  return static_cast<int>(((max_pos / block_size + 1) + 15) / 16 * 16);
+  return (index_blocks(max_pos, block_size) + 15) / 16 * 16;
 }
 
 int select_bank_cap(int topk) {
@@ -1260,17 +1265,20 @@ int select_bank_cap(int topk) {
 
 hipError_t launch_lightning_indexer(const int32_t* image, int seq_len, const void* index_q,
                                     const void* index_k, int32_t* block_idx, float* scores,
-                                    int block_stride, int num_heads, int head_dim,
-                                    int block_size, int topk, int local_blocks,
+                                    int num_blocks, int block_stride, int num_heads,
+                                    int head_dim, int block_size, int topk, int local_blocks,
                                     int init_blocks, float scale, int shift, int row_mask,
                                     hipStream_t stream) {
   if (seq_len <= 0) return hipSuccess;
   if (head_dim != 128 || num_heads != 4) return hipErrorInvalidValue;
-  dim3 grid((block_stride + 3) / 4, seq_len);
+  // No wave past the last block of the longest context: those of the stride's
+  // padding cost their start (1,000 tokens on up to 200 keys, 14 of 16 waves: 60.6
+  // us with the selection, without them 16.1).
+  dim3 grid((num_blocks + 3) / 4, seq_len);
   const auto* iq = static_cast<const uint16_t*>(index_q);
   const auto* ik = static_cast<const uint16_t*>(index_k);
   if (row_mask + 1 >= 64 && block_size % 64 == 0) {
-    hipLaunchKernelGGL((index_scores_rounds_kernel<128, 4>), dim3(block_stride, seq_len),
+    hipLaunchKernelGGL((index_scores_rounds_kernel<128, 4>), dim3(num_blocks, seq_len),
                        dim3(64), 0, stream, image, iq, ik, scores, block_stride, block_size,
                        scale, shift, row_mask);
   } else if (row_mask + 1 >= 64)

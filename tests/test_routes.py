@@ -1,8 +1,11 @@
 """Which kernel a full-attention token plan takes, and with how many workgroups
 (host rules; no GPU is touched)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+from inferno_amd._lib import I64, P_I64, lib
 from inferno_amd.kv import FULL, AttentionPlan, KVRunTable
 from tests.helpers import (ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, ROUTE_PAIR, bf16_route,
                            make_prefill_case)
@@ -57,3 +60,14 @@ def test_narrow_workgroups_cover_every_token(head_dim, num_kv, gqa, tokens):
 def test_a_tie_goes_to_the_query_blocks():
     plan = token_plan([25] * 300, [20] * 300, num_kv=1)
     assert bf16_route(plan, 2, 1, 256) == (ROUTE_PAIR, 0)
+
+
+@pytest.mark.parametrize("top,block_size,blocks", [(0, 64, 1), (63, 64, 1), (64, 64, 2), (199, 128, 2),
+                                                   (131071, 128, 1024)])
+def test_index_waves_end_with_the_longest_context(top, block_size, blocks):
+    """The scores' rows are padded to 16 blocks; the padding gets no waves."""
+    plan = token_plan([0, top], [1, 1], page_len=128)
+    fn = lib().ifr_internal_index_blocks
+    fn.restype, fn.argtypes = C.c_int64, [P_I64, I64]
+    assert fn(plan.info_ptr, block_size) == blocks
+    assert lib().ifr_index_scores_bytes(plan.info_ptr, 4, block_size) == 2 * 4 * 4 * (-(-blocks // 16) * 16)
