@@ -1396,6 +1396,12 @@ int64_t ifr_gemm_cols_workspace_bytes(int64_t rows, int64_t cols, int64_t seq_le
   return ifr::gemm_cols_workspace_bytes(seq_len, rows, cols);
 }
 
+// Not part of the C API, for the tests: gemm_cols_plan.
+void ifr_internal_gemm_plan(int64_t rows, int64_t cols, int64_t seq_len, int64_t workspace_bytes,
+                            int64_t* plan) {
+  ifr::gemm_cols_plan(seq_len, rows, cols, workspace_bytes, plan);
+}
+
 int32_t ifr_dispatch_gemm_cols(const void* x, const void* weight, void* output, int64_t rows,
                                int64_t cols, int64_t seq_len, void* workspace,
                                int64_t workspace_bytes, uint64_t stream) {

@@ -465,6 +465,15 @@ int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return splits > 1 ? splits * M * N * 4 : 0;
 }
 
+void gemm_cols_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int64_t* plan) {
+  const int span = decode_span(M, K);
+  const TilePlan p = span ? TilePlan{0, 0, static_cast<int>(K / span)}
+                          : tile_plan(M, N, K, workspace_bytes);
+  plan[0] = p.bm;
+  plan[1] = p.bn;
+  plan[2] = p.splits;
+}
+
 // Batches of more than 256 tiles of 64 x 64 run without a workspace, fewer with
 // room for two splits; what the plan takes beyond that is a matter of speed (400
 // tokens x 2816 x 8192: four splits 33.8 us, two 32.4, none 41.1).

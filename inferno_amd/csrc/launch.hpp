@@ -121,6 +121,8 @@ hipError_t launch_bq_block_quant(const void* src, void* x_i8, float* x_sa, int64
 // fastest plan uses, _required_bytes what the launch cannot do without.
 int64_t gemm_cols_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int64_t gemm_cols_required_bytes(int64_t M, int64_t N, int64_t K);
+// {tile tokens, tile columns, k slices} of a launch; a decode batch has no tile.
+void gemm_cols_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int64_t* plan);
 hipError_t launch_gemm_cols(const void* x, const void* w, void* out, float* workspace,
                             int64_t workspace_bytes, int64_t M, int64_t N, int64_t K,
                             hipStream_t stream);

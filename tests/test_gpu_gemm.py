@@ -61,20 +61,32 @@ def test_gemm_cols_integer_operands_bit_exact(seq, rows, cols):
     assert np.array_equal(got, want)
 
 
-# Sizes around every tile shape of the batched kernel (64, 128, 192 and 256
-# tokens by 64 or 128 columns), its k splits and its three-chunk loop (2, 4, 6
-# and 64 chunks): integer operands, so every sum is exact in any order.
-@pytest.mark.parametrize("seq,rows,cols", [(65, 16, 128), (65, 2816, 4096), (127, 144, 256),
-                                           (129, 80, 384), (193, 2816, 512), (500, 2816, 4096),
-                                           (769, 2816, 256), (1537, 2816, 128),
-                                           (2000, 2816, 384), (4099, 1040, 128)])
+# Batches past the decode sizes and the plan each takes with its workspace: tile
+# tokens, tile columns, k slices.  Every tile shape with and without slices; ragged
+# last tiles in both directions; 2, 4, 6, 16, 64 and 128 chunks of the loop (three
+# chunks deep); one to three bands of token tiles.  The plans themselves are checked
+# without a GPU (test_routes.py).
+TILE_CASES = {
+    (65, 16, 128): (64, 64, 1), (127, 144, 256): (64, 64, 1), (129, 80, 384): (64, 64, 1),
+    (193, 2816, 512): (64, 64, 1), (65, 272, 2048): (64, 64, 4),
+    (500, 2816, 4096): (128, 64, 1), (65, 2816, 4096): (128, 64, 4),
+    (769, 2816, 256): (128, 128, 1), (1933, 272, 4096): (128, 128, 4),
+    (1537, 2816, 128): (192, 128, 1), (2000, 2816, 384): (192, 128, 1),
+    (4099, 1040, 128): (192, 128, 1), (324, 2816, 8192): (192, 128, 4),
+    (2137, 2816, 256): (256, 128, 1), (1175, 5376, 256): (256, 128, 1),
+    (398, 2816, 8192): (256, 128, 4),
+}
+
+
+@pytest.mark.parametrize("seq,rows,cols", TILE_CASES)
 def test_gemm_cols_tiles_bit_exact(seq, rows, cols):
+    """Integer operands, so every sum is exact in any order."""
     announce(f"gemm_cols tiles seq={seq} rows={rows} cols={cols}")
     rng = np.random.default_rng(seq + rows + cols)
     x = rng.integers(-3, 4, (seq, cols)).astype(np.float32)
     w = rng.integers(-3, 4, (rows, cols)).astype(np.float32)
     got = _run(_bf(x), _bf(w), seq, rows, cols)
-    # |sum| <= 9 * 4096: exact in f32, and one rounding to bf16 in the oracle's conversion.
+    # |sum| <= 9 * 8192: exact in f32, and one rounding to bf16 in the oracle's conversion.
     assert np.array_equal(got, oracle.f32_to_bf16((x @ w.T).ravel()).reshape(seq, rows))
 
 

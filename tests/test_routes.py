@@ -1,5 +1,5 @@
-"""Which kernel a full-attention token plan takes, and with how many workgroups
-(host rules; no GPU is touched)."""
+"""Which kernel a full-attention token plan or an o_proj batch takes, and with how many
+workgroups (host rules; no GPU is touched)."""
 import ctypes as C
 
 import numpy as np
@@ -71,3 +71,33 @@ def test_index_waves_end_with_the_longest_context(top, block_size, blocks):
     fn.restype, fn.argtypes = C.c_int64, [P_I64, I64]
     assert fn(plan.info_ptr, block_size) == blocks
     assert lib().ifr_index_scores_bytes(plan.info_ptr, 4, block_size) == 2 * 4 * 4 * (-(-blocks // 16) * 16)
+
+
+def gemm_plan(rows, cols, seq_len, workspace_bytes):
+    fn = lib().ifr_internal_gemm_plan
+    fn.restype, fn.argtypes = None, [I64, I64, I64, I64, P_I64]
+    plan = (C.c_int64 * 3)()
+    fn(rows, cols, seq_len, workspace_bytes, plan)
+    return tuple(plan)
+
+
+def test_the_gemm_tests_cover_every_tile_kernel():
+    from tests.test_gpu_gemm import TILE_CASES
+
+    for (seq, rows, cols), plan in TILE_CASES.items():
+        bytes_ = lib().ifr_gemm_cols_workspace_bytes(rows, cols, seq)
+        assert gemm_plan(rows, cols, seq, bytes_) == plan, (seq, rows, cols)
+        assert bytes_ == (plan[2] * seq * rows * 4 if plan[2] > 1 else 0)
+    shapes = [(64, 64), (128, 64), (128, 128), (192, 128), (256, 128)]
+    assert {(m, n, s > 1) for m, n, s in TILE_CASES.values()} == {
+        (m, n, split) for m, n in shapes for split in (False, True)}
+
+
+@pytest.mark.parametrize("seq,cols,slices", [(1, 4096, 16), (16, 256, 1), (16, 4096, 16), (16, 4608, 9),
+                                             (1, 8192, 16), (17, 4096, 8), (64, 8192, 16)])
+def test_decode_batches_slice_k(seq, cols, slices):
+    """Slices of 256 up to 16 tokens and k of 4,096 (joined in the workgroup, no
+    workspace), of 512 past either."""
+    assert gemm_plan(2816, cols, seq, 1 << 40) == (0, 0, slices)
+    joined = seq <= 16 and cols <= 4096
+    assert lib().ifr_gemm_cols_workspace_bytes(2816, cols, seq) == (0 if joined else slices * seq * 2816 * 4)
