@@ -1,7 +1,9 @@
 """GPU parity of chunked prefill over the paged cache (full attention):
 append of the chunk (RoPE + cache write, bit-exact), then the MFMA prefill
 kernel against the oracle's token-partitioned route
-(FlashPrefillFullKernel + PrefillMergeKernel) within 1e-2 / one bf16 spacing."""
+(FlashPrefillFullKernel + PrefillMergeKernel) within 1e-2 / one bf16 spacing.
+Which kernel that is depends on the chunk's rows and the page size;
+test_gpu_prefill_narrow.py names the kernel of each of its cases."""
 import numpy as np
 import pytest
 

@@ -7,7 +7,9 @@ oracle's token-partitioned route, within 1e-2 (one bf16 spacing where
 16 tokens, so the cases cover partial blocks, waves without live rows, the
 causal diagonal, page-table windows that move, and both of the kernel's
 block placements (kv head counts that divide the 8 XCDs and one that does
-not)."""
+not).  Chunks of few rows over pages of 16 rows and more take the narrow kernel,
+so the short cases here run that one; test_gpu_prefill_narrow.py names the
+kernel of each of its cases."""
 import numpy as np
 import pytest
 

@@ -340,3 +340,38 @@ def test_block_and_round_edges(block, page_len, topk):
                                         num_kv=NUM_KV, head_dim=HD, kv_stride=KV_STRIDE,
                                         block_size=block, topk=topk, page_len=page_len, seq_len=n)
     assert_bar(compare_bf16(from_dev(out, np.uint16), ref), f"sparse edges block={block}")
+
+
+@pytest.mark.parametrize("gap", [8, 512])
+def test_block_sparse_rows_wider_than_their_heads(gap):
+    """Cache rows further apart than num_kv * head_dim, NaN between them and past
+    each sequence's last position; every block of each context."""
+    announce(f"sparse kv_stride gap={gap}")
+    rng = np.random.default_rng(gap)
+    n, page_len = len(EDGE_CTX), 64
+    kvs = KV_STRIDE + gap
+    case = make_decode_case(33, EDGE_CTX, page_len=page_len)
+    used = np.zeros(case.cache_rows, dtype=bool)
+    for pages, c in zip(case.pages, EDGE_CTX):
+        used[np.concatenate([np.arange(page_len) + g * page_len for g in pages])[:c + 1]] = True
+    q = _bf(rng.standard_normal(n * NUM_Q * HD) / np.sqrt(HD))
+    k, v = (_bf(rng.standard_normal(case.cache_rows * kvs)) for _ in "kv")
+    blocks = np.full((n, IH, TOPK + 1), -1, dtype=np.int32)
+    for i, c in enumerate(EDGE_CTX):
+        blocks[i, :, :c // BLOCK + 1] = np.arange(c // BLOCK + 1)
+
+    def poisoned(x):
+        x = x.reshape(case.cache_rows, kvs).copy()
+        x[~used] = 0x7FC0
+        x[:, KV_STRIDE:] = 0x7FC0
+        return to_dev(x)
+
+    out = empty_dev(n * NUM_Q * HD, np.uint16)
+    A.dispatch_block_sparse_attention(_plan(case.runs, case.base_rows, n, case.cache_rows, page_len),
+                                      to_dev(q), poisoned(k), poisoned(v), to_dev(blocks), out,
+                                      kv_stride=kvs, topk_blocks=TOPK + 1)
+    ref = oracle.block_sparse_attention(case.runs, case.base_rows, q, k, v, blocks, num_q=NUM_Q,
+                                        num_kv=NUM_KV, head_dim=HD, kv_stride=kvs,
+                                        block_size=BLOCK, topk=TOPK + 1, page_len=page_len,
+                                        seq_len=n)
+    assert_bar(compare_bf16(from_dev(out, np.uint16), ref), f"sparse kv_stride gap={gap}")
