@@ -36,6 +36,10 @@
 // far inside the bf16 output tolerance, and it saves a third of the
 // softmax's VALU work, which bounds this kernel together with the MFMAs.
 //
+// bf16 plans come here where a 16-key tile may leave its page (pages of 8 rows and
+// fewer) and for rows of more than 2^25 elements; the others take the kernels of
+// prefill_pair.hip and prefill_narrow.hip.
+//
 // K and V reach LDS straight from global memory (global_load_lds_dwordx4,
 // no registers) one iteration ahead.  K rows are stored XOR-swizzled (16-byte
 // chunk c of key k at position c ^ (k & 15)) so the 16 keys a QK operand read
@@ -250,54 +254,32 @@ void prefill_full_mfma_kernel(
           (lds_void_t*)(vdst + lds_row * kRowBytes), 16, 0, 0);
     }
   };
-  // The same for an iteration whose kStageRows rows per wave all lie below
+  // bq: the same for an iteration whose kStageRows rows per wave all lie below
   // count_max and inside one page (pages of >= 16 rows): one page lookup, a
   // wave-uniform row base and per-lane byte offsets fixed for the kernel.
-  // Row rr = 2i + half of the wave's rows sits rr * kv_stride * 2 bytes past
-  // the base, i.e. i * 4 * kv_stride (uniform) + hk (lane); its K chunk
-  // row ^ rr = (row ^ half) ^ 2i gives the byte offset x16 ^ 32i, its V
-  // chunk row ^ 2*(rr & 3) one of two lane constants (i even or odd).
-  // bq: row rr = 4i + lr (lr = lane / 16) at i * 4 * kv_stride + lr *
-  // kv_stride bytes, K chunk (c ^ lr) ^ 4i.
+  // Row rr = 4i + lr of the wave's rows (lr = lane / 16) sits i * 4 * kv_stride
+  // (uniform) + lr * kv_stride (hk) bytes past the base, its K chunk at
+  // (c ^ lr) ^ 4i.
   const int lr = lane >> 4;
   const int cq = lane & 15;
-  const int hk = kBq ? lr * static_cast<int>(kv_stride) : half * static_cast<int>(kv_stride) * 2;
-  const uint32_t x16 = kBq ? 16u * static_cast<uint32_t>(cq ^ lr)
-                           : 16u * static_cast<uint32_t>(row ^ half);
-  const uint32_t hv0 = kBq ? static_cast<uint32_t>(hk) + 16u * static_cast<uint32_t>(cq)
-                           : static_cast<uint32_t>(hk) + 16u * static_cast<uint32_t>(row ^ (2 * half));
-  const uint32_t hv1 =
-      static_cast<uint32_t>(hk) + 16u * static_cast<uint32_t>(row ^ (4 + 2 * half));
-  auto stage_page = [&](int it, uint8_t* kdst, uint8_t* vdst, int buf) {
+  const int hk = lr * static_cast<int>(kv_stride);
+  const uint32_t x16 = 16u * static_cast<uint32_t>(cq ^ lr);
+  const uint32_t hv = static_cast<uint32_t>(hk) + 16u * static_cast<uint32_t>(cq);
+  auto stage_page = [&](int it, uint8_t* kdst, int buf) {
     const int key0 = it * kKeys + wave * kStageRows;  // wave-uniform
     const int prow = __builtin_amdgcn_readfirstlane(page_rows[(key0 >> shift) - wbase]);
     const int64_t slot0 = static_cast<int64_t>(prow) + (key0 & row_mask);
-    if constexpr (kBq) {
-      const char* kb = reinterpret_cast<const char*>(kbase8 + slot0 * kv_stride);
-      const char* vb = reinterpret_cast<const char*>(vbase8 + slot0 * kv_stride);
-      const int64_t step = 4 * kv_stride;
+    const char* kb = reinterpret_cast<const char*>(kbase8 + slot0 * kv_stride);
+    const char* vb = reinterpret_cast<const char*>(vbase8 + slot0 * kv_stride);
+    const int64_t step = 4 * kv_stride;
 #pragma unroll
-      for (int i = 0; i < kStageRows / 4; ++i) {
-        __builtin_amdgcn_global_load_lds(
-            kb + i * step + (static_cast<uint32_t>(hk) + (x16 ^ (64u * i))),
-            (lds_void_t*)(kdst + (wave * kStageRows + 4 * i) * kBqRowBytes), 16, 0, 0);
-        vcodes[i] = *reinterpret_cast<const uint4*>(vb + i * step + hv0);
-      }
-      stage_scales(it, buf);
-      return;
+    for (int i = 0; i < kStageRows / 4; ++i) {
+      __builtin_amdgcn_global_load_lds(
+          kb + i * step + (static_cast<uint32_t>(hk) + (x16 ^ (64u * i))),
+          (lds_void_t*)(kdst + (wave * kStageRows + 4 * i) * kBqRowBytes), 16, 0, 0);
+      vcodes[i] = *reinterpret_cast<const uint4*>(vb + i * step + hv);
     }
-    const char* kb = reinterpret_cast<const char*>(kbase + slot0 * kv_stride);
-    const char* vb = reinterpret_cast<const char*>(vbase + slot0 * kv_stride);
-    const int64_t step = 4 * kv_stride;  // bytes from row pair i to i + 1
-#pragma unroll
-    for (int i = 0; i < kStageRows / 2; ++i) {
-      const int lds_row = wave * kStageRows + 2 * i;  // wave-uniform
-      const uint32_t ko = static_cast<uint32_t>(hk) + (x16 ^ (32u * i));
-      __builtin_amdgcn_global_load_lds(kb + i * step + ko,
-                                       (lds_void_t*)(kdst + lds_row * kRowBytes), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(vb + i * step + ((i & 1) ? hv1 : hv0),
-                                       (lds_void_t*)(vdst + lds_row * kRowBytes), 16, 0, 0);
-    }
+    stage_scales(it, buf);
   };
   // After the wave's loads have landed: bf16 zeroes the V rows of keys past
   // count_max; bq writes its V codes as bf16 rows (the bf16 swizzle: chunk c
@@ -380,19 +362,6 @@ void prefill_full_mfma_kernel(
   // ((raw - qi_bias) * f_q) * k_scale / 127^2 per (row, key), raw the
   // integer dot plus 128 * sum q; value 4j + i holds key 8j + 4*half + i.
   constexpr int kKAhead = 6;
-  // bf16 page staging split into 16 single loads (K then V of row pair i
-  // for load j = 2i, 2i + 1), so they can be issued between MFMAs.
-  auto page_load = [&](int j, const char* kb, const char* vb, uint8_t* kdst, uint8_t* vdst) {
-    const int i = j >> 1;
-    const int64_t step = 4 * kv_stride;  // bytes from row pair i to i + 1
-    const int lds_row = wave * kStageRows + 2 * i;  // wave-uniform
-    if ((j & 1) == 0)
-      __builtin_amdgcn_global_load_lds(kb + i * step + (static_cast<uint32_t>(hk) + (x16 ^ (32u * i))),
-                                       (lds_void_t*)(kdst + lds_row * kRowBytes), 16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds(vb + i * step + ((i & 1) ? hv1 : hv0),
-                                       (lds_void_t*)(vdst + lds_row * kRowBytes), 16, 0, 0);
-  };
   auto qk = [&](const uint8_t* kl, int h, int buf) {
     if constexpr (kBq) {
       i32x16_t si;
@@ -447,38 +416,6 @@ void prefill_full_mfma_kernel(
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
     __builtin_amdgcn_sched_group_barrier(0x008, kKAhead, 0);
-    return sblk;
-  };
-  // bf16 S^T of tile pair h with the next iteration's page-staged loads
-  // 8h .. 8h + 7 issued after the odd MFMAs: a load's issue then overlaps
-  // the MFMA pipe instead of holding up the wave ahead of the scores (the
-  // 64 staging loads of a block take about a thousand cycles to pass the
-  // texture unit).
-  auto qk_staging = [&](const uint8_t* kl, int h, const char* kb, const char* vb,
-                        uint8_t* kdst, uint8_t* vdst) {
-    f32x16_t sblk;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) sblk[v] = 0.0f;
-    const uint8_t* kh = kl + 32 * h * kRowBytes;
-    uint4 kf[kPD / 16];
-#pragma unroll
-    for (int d = 0; d < kKAhead; ++d)
-      kf[d] = *reinterpret_cast<const uint4*>(kh + (k_lane ^ (32 * d)));
-#pragma unroll
-    for (int d = 0; d < kPD / 16; ++d) {
-      if (d + kKAhead < kPD / 16)
-        kf[d + kKAhead] = *reinterpret_cast<const uint4*>(kh + (k_lane ^ (32 * (d + kKAhead))));
-      sblk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kf[d]), qf[d],
-                                                     sblk, 0, 0, 0);
-      if (d & 1) page_load(8 * h + (d >> 1), kb, vb, kdst, vdst);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x100, kKAhead, 0);
-#pragma unroll
-    for (int d = 0; d < kPD / 16; ++d) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (d + kKAhead < kPD / 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      if (d & 1) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
-    }
     return sblk;
   };
   // Online softmax of the pair's two tiles; tile_key0 is the first key of
@@ -650,25 +587,19 @@ void prefill_full_mfma_kernel(
   auto full_iteration = [&](bool page_stage, int it, const uint8_t* kl, const uint8_t* vl,
                             uint8_t* knext, uint8_t* vnext) {
     const int buf = it & 1;
-    f32x16_t s0, s1;
-    if (!kBq && page_stage) {  // block-uniform
-      // One page lookup for the wave's rows of the next iteration; the
-      // loads go out between the score MFMAs.
-      const int key0 = (it + 1) * kKeys + wave * kStageRows;  // wave-uniform
-      const int prow = __builtin_amdgcn_readfirstlane(page_rows[(key0 >> shift) - wbase]);
-      const int64_t slot0 = static_cast<int64_t>(prow) + (key0 & row_mask);
-      const char* kb = reinterpret_cast<const char*>(kbase + slot0 * kv_stride);
-      const char* vb = reinterpret_cast<const char*>(vbase + slot0 * kv_stride);
-      s0 = qk_staging(kl, 0, kb, vb, knext, vnext);
-      s1 = qk_staging(kl, 1, kb, vb, knext, vnext);
-    } else {
+    if constexpr (kBq) {
       if (page_stage)  // block-uniform
-        stage_page(it + 1, knext, vnext, buf ^ 1);
+        stage_page(it + 1, knext, buf ^ 1);
       else
         stage(it + 1, knext, vnext, buf ^ 1);
-      s0 = qk(kl, 0, buf);
-      s1 = qk(kl, 1, buf);
+    } else {
+      stage(it + 1, knext, vnext, buf ^ 1);
+      // The loads go out ahead of the scores: between their MFMAs the address math of
+      // 8-row pages costs up to 2 %.
+      __builtin_amdgcn_sched_barrier(0);
     }
+    const f32x16_t s0 = qk(kl, 0, buf);
+    const f32x16_t s1 = qk(kl, 1, buf);
     // Straight-line order that lets the pair-1 scores (MFMA) run under the
     // pair-0 softmax (VALU), and the pair-0 PV (MFMA) under the pair-1
     // softmax.
@@ -707,7 +638,7 @@ void prefill_full_mfma_kernel(
   const int block_min = ntok == kPTokens ? base_pos + (t0 - buf_start) + 1 : 0;
   const int it_full = min(n_iters, block_min / kKeys) & ~1;
   int it = 0;
-  // A staged iteration below it_full has every row below count_max, so with
+  // bq: a staged iteration below it_full has every row below count_max, so with
   // pages of >= 16 rows it stages through stage_page.
   const bool pages16 = shift >= 4;
   for (; it < it_full; it += 2) {

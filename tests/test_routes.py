@@ -7,8 +7,8 @@ import pytest
 
 from inferno_amd._lib import I64, P_I64, lib
 from inferno_amd.kv import FULL, AttentionPlan, KVRunTable
-from tests.helpers import (ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, ROUTE_PAIR, bf16_route,
-                           make_prefill_case)
+from tests.helpers import (ROUTE_FULL, ROUTE_NARROW_PAIRS, ROUTE_NARROW_TILES, ROUTE_PAIR,
+                           ROUTE_WIDE, bf16_route, make_prefill_case)
 
 
 def token_plan(prefix, new, page_len=64, num_kv=8, head_dim=256):
@@ -101,3 +101,13 @@ def test_decode_batches_slice_k(seq, cols, slices):
     assert gemm_plan(2816, cols, seq, 1 << 40) == (0, 0, slices)
     joined = seq <= 16 and cols <= 4096
     assert lib().ifr_gemm_cols_workspace_bytes(2816, cols, seq) == (0 if joined else slices * seq * 2816 * 4)
+
+
+@pytest.mark.parametrize("page_len,kv_stride", [(8, None), (64, (1 << 25) + 8)])
+def test_small_pages_and_wide_rows_take_the_query_blocks(page_len, kv_stride):
+    """A tile that may leave its page, and row offsets past 32 bits, stay with the
+    kernels that look every row up."""
+    for new in ([1, 40], [700, 300]):
+        plan = token_plan([100, 100], new, page_len=page_len)
+        assert bf16_route(plan, 16, 8, 256, kv_stride) == (ROUTE_FULL, 0)
+        assert bf16_route(plan, 16, 2, 512, kv_stride) == (ROUTE_WIDE, 0)
