@@ -330,7 +330,9 @@ int32_t ifr_bq_block_sparse_attention(
  * seq_len splits the contraction over workgroups into f32 partials in
  * `workspace` (ifr_gemm_cols_workspace_bytes; 0 means none is needed).  Past 64
  * tokens a smaller workspace, or none where the output has more than 256 tiles of
- * 64 x 64, runs with the splits that fit it. */
+ * 64 x 64, runs with the splits that fit it; the splits are added in order, so
+ * there the bits of a result depend on the size of the workspace that is passed
+ * (f32 sums in another order), and are the same for the same size. */
 int64_t ifr_gemm_cols_workspace_bytes(int64_t rows, int64_t cols, int64_t seq_len);
 int32_t ifr_dispatch_gemm_cols(const void* x, const void* weight, void* output,
                                int64_t rows, int64_t cols, int64_t seq_len,

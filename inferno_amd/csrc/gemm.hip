@@ -413,7 +413,10 @@ hipError_t launch_tile(const uint16_t* x, const uint16_t* w, uint16_t* out, floa
 // their own start and the f32 partials' way out and back.  It picks the
 // measured best or one within 5 % of it (12 % at 128 tokens): 128 x 64 22.2 us at
 // 500 tokens (two splits of 128 x 128 21.8), 192 x 128 45.1 us at 2,000 (242 of 256 CUs;
-// 256 x 128, 176 tiles, 47.9), 256 x 128 342 us at 16,384 (1,106 TFLOP/s).
+// 256 x 128, 176 tiles, 47.9), 256 x 128 342 us at 16,384 (1,106 TFLOP/s).  Other N
+// and K were not fitted but measured, 65 to 6,000 tokens against the 64 x 64 kernel
+// before it: 1.05 to 4.7 times as fast at N = 1,024 x 2,048, 1.3 to 4.5 at 512 x 4,096,
+// 1.4 to 4.0 at 272 x 8,192, 3.1 to 6.2 at 5,376 x 8,192, 2.5 to 4.1 at 16,384 x 1,024.
 // Splits whose partials do not fit the caller's workspace are left out.
 struct TilePlan {
   int bm, bn, splits;

@@ -22,20 +22,22 @@
 // barrier; the two barriers of an iteration publish the maxima and the weights.
 //
 // What bounds them is instruction issue: a lone wave of a SIMD issues about one
-// instruction per 5 cycles and one LDS read per 24 to 34.  Hence two kernels.
+// instruction per 5 cycles and one LDS read per 24 to 34 (counted, 500 tokens on 7,013
+// keys, pairs: a wave's cycles go to issuing by 51 %, to waits by 29 %, to waiting for
+// the issue by 20 %; matrix cores busy 20 %).  Hence two kernels.
 // prefill_narrow_pairs_kernel (head_dim 256) takes tile pairs on
 // v_mfma_f32_32x32x16_bf16, 128 keys an iteration: the fewest instructions per
 // key, but its LDS fills a CU.  prefill_narrow_tiles_kernel takes single tiles
 // on v_mfma_f32_16x16x32_bf16, 64 keys an iteration: two blocks fit a CU at
 // head_dim 256 and run under each other's waits.
 //
-// Measured at 16 q / 8 kv heads x 256 (us, prefill_pair_kernel / pairs / tiles;
-// prefill_full_mfma_kernel): 64 tokens on 7,000 270 / 134 / 185; 296.  500 on
-// 7,013 284 / 140 / 192; 484.  1,000 on 7,000 313 / 278 / 250; 513.  2,000 on
-// 7,000 361 / 580 / 505; 552.  32 tokens decoding at 3,000 beside a 512-token
-// chunk 278 / 191 / 157; 374.  At 16 / 2 x 512
-// (query-block kernel / tiles): 64 tokens 518 / 275; 500 690 / 300; 1,000 750 /
-// 580; 2,000 671 / 1,230; the mixed step 630 / 290.
+// Measured on one card at 16 q / 8 kv heads x 256 (us, prefill_pair_kernel / pairs /
+// tiles; prefill_full_mfma_kernel): 64 tokens on 7,000 271 / 136 / 186; 297.  500 on
+// 7,013 284 / 140 / 186; 483.  1,000 on 7,000 304 / 282 / 238; 513.  2,000 on
+// 7,000 370 / 591 / 491; 552.  32 tokens decoding at 3,000 beside a 512-token
+// chunk 261 / 215 / 159; 371.  At 16 / 2 x 512
+// (query-block kernel / tiles): 64 tokens 517 / 278; 500 691 / 293; 1,000 749 /
+// 583; 2,000 673 / 1,233; the mixed step 624 / 298.
 #include <algorithm>
 #include <type_traits>
 

@@ -7,7 +7,8 @@
 // A row is one (query token, q head).  prefill_full_mfma_kernel gives a wave 32
 // rows and all 256 output dims, 200 registers of accumulators and queries, so a
 // SIMD holds one wave, and that wave pays for its LDS reads, its softmax and its
-// MFMAs one after the other (7,400 cycles for 64 keys, 2,640 of them MFMA).
+// MFMAs one after the other (7,400 cycles for 64 keys where one round of blocks runs,
+// 6,450 on a full grid).
 // Here two waves share the 32 rows of a row group:
 //
 //   scores   wave w of the pair takes keys 32 w .. +31 of the 64 staged ones (two
@@ -31,11 +32,14 @@
 // barrier 3 it + 3.  V has two buffers: V of it + 1 is loaded from barrier 3 it + 1,
 // when V of it - 1 has no reader left, and is waited for before 3 it + 3 as well.
 //
-// Bound by the three phases' own chains (5,500 cycles for 64 keys, of which 2,100
-// MFMA on each SIMD at a lo part in every other tile).  Measured, 8 kv heads, from
-// prefill_full_mfma_kernel: 2,000 tokens on 7,000 keys 525 -> 361 us, two chunks
-// of 1,500 451 -> 377 us, eight of 2,048 2,962 -> 2,888 us.  A V load that is
-// issued after P.V instead costs 10 to 20 %, waves in step 8 %.
+// Bound by the three phases' own chains: 5,500 cycles for 64 keys in one round of
+// blocks, 5,930 on a full grid, the matrix cores busy for 40 % of them (a lo part in
+// about every third tile).  On the full grid the clock falls with the cycles (2.31 to
+// 2.17 GHz), which gives most of the gain back.  Measured on one card, 8 kv heads, from
+// prefill_full_mfma_kernel: 2,000 tokens on 7,000 keys 552 -> 370 us, two chunks of
+// 1,500 on 1,000 to 8,000 420 -> 376, four of 500 on 1,000 111 -> 77, 2,100 on 100
+// 154 -> 98, eight of 2,048 on up to 16,384 3,042 -> 2,951.  A V load that is issued
+// after P.V instead costs 10 to 20 %, waves in step 8 %.
 #include <type_traits>
 
 #include "launch.hpp"

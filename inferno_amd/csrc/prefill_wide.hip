@@ -301,7 +301,10 @@ void prefill_wide_mfma_kernel(
   // The Q^T fragments are waited for here.  Otherwise the compiler moves their
   // loads past the wait, carries them as outstanding into the loop, and puts a
   // vmcnt(0) among the score MFMAs of every iteration, right behind the first
-  // staging load of the next one.
+  // staging load of the next one.  Not a gain everywhere: 8 x 2,048 tokens at one kv
+  // head 2,564 -> 2,489 us, 2,048 on none 178 -> 176, 2 x 1,500 on 1,000 to 8,000 keys
+  // 708 -> 700; 4 x 513 on up to 2,000 206 -> 209, 8 x 513 at one kv head 243 -> 247;
+  // over 24 such shapes nothing on average.
 #pragma unroll
   for (int d = 0; d < kQFrags; ++d) asm volatile("" : "+v"(qf[d]));
   if (n_iters > 0) land_v(0, vbuf0);

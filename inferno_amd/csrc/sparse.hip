@@ -994,7 +994,7 @@ __global__ __launch_bounds__(256) void bq_sparse_kernel(
 }
 
 // The batched route of bq_sparse_kernel (one sequential pass per (token, kv
-// head)) with the bf16 kernel's split: four waves per (token, kv head), each
+// head)), split by output dims: four waves per (token, kv head), each
 // forming the same int8 scores (exact integers, so identical) and owning 32
 // of the 128 output dims, with kSAhead tiles in flight in rotating register
 // sets.  One wave per (token, kv head) left three quarters of the SIMDs idle
@@ -1056,8 +1056,8 @@ __global__ __launch_bounds__(256) void bq_sparse_split_kernel(
   const int8_t* vh = v_base + static_cast<int64_t>(h) * kSD + kSDW * dq;
   const int32_t* brow = block_idx + static_cast<int64_t>(row) * topk;
   // V staging: lane takes 8 bytes (dims 8*(l%4) ..) of the wave's 32 dims of
-  // row l/4 and writes them as 8 bf16 (exact); the transposing read as in
-  // sparse_attention_kernel.
+  // row l/4 and writes them as 8 bf16 (exact).  Transposing read: lane r16 of group
+  // g addresses row 4g + r16/4, dims 4*(r16%4) .. +3.
   const int vrow_l = lane >> 2;
   const int vcol = 8 * (lane & 3);
   const int tr_off = (4 * g + (r16 >> 2)) * kSVPitchW + 8 * (r16 & 3);
@@ -1174,9 +1174,9 @@ __global__ __launch_bounds__(256) void bq_sparse_split_kernel(
     }
   };
 
-  // Rotating register sets as in sparse_attention_kernel: unconditional
-  // loads (past the block list they read the sequence's first row), leaving
-  // the loop the only branch, page rows read one step ahead.
+  // Rotating register sets: unconditional loads (past the block list they read
+  // the sequence's first row), leaving the loop the only branch, page rows read
+  // one step ahead.
   auto advance = [&](const TileCursor& c) {
     return c.valid ? next_tile(c, brow, topk, block_size, cap) : c;
   };
