@@ -1,9 +1,10 @@
-"""What the kernels' own waits and launch bounds rest on, in the gfx950 code that the
-compiler makes of them.  The workgroup barriers of the kernels that write their own (inline `s_barrier`
-instead of __syncthreads, so that loads in flight stay in flight), in the gfx950
-code that the compiler makes of them: on every path, no LDS access of the wave may
-still be outstanding when it arrives.  Another wave may overwrite that LDS right
-after the barrier; a load that only lands late is not an order."""
+"""What the kernels rest on in the gfx950 code that the compiler makes of them.
+
+The kernels that write their own workgroup barrier (inline `s_barrier` instead of
+__syncthreads, so that loads in flight stay in flight): on every path, no LDS access of
+the wave may still be outstanding when it arrives.  Another wave may overwrite that LDS
+right after the barrier; that a load lands late is not an order.  The GEMM kernels: no
+operand spills to scratch."""
 import re
 import subprocess
 
